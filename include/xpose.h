@@ -408,9 +408,9 @@ typedef struct {
      * shape or device does not allow it). */
     int32_t  exec_mode;
     /* How xp_session_prefill runs a prompt of n >= 3 tokens: XP_PREFILL_AUTO
-     * (the first n - 1 tokens through the batched M = 16 step, 16 positions
-     * per pass on the session's KV cache, then the last token on the
-     * session's own path) or XP_PREFILL_TOKENS (one token step per token,
+     * (the first n - 1 tokens together on the session's KV cache, up to 16 in
+     * one pass of the batched step, more as GEMMs over up to 2048 positions a
+     * pass, then the last token on the session's own path) or XP_PREFILL_TOKENS (one token step per token,
      * the reference's decode-shaped prefill, decode.cpp:1785-1815). */
     int32_t  prefill_mode;
     /* Where the persistent token kernel runs its exchanges: XP_PLACE_AUTO

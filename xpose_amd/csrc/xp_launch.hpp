@@ -333,6 +333,86 @@ struct PrefillBatch;
 PrefillBatch* prefill_batch_create(const xp_session* s);
 int prefill_batch_run(PrefillBatch* p, const uint32_t* ids, uint32_t n, uint32_t pos0);
 void prefill_batch_destroy(PrefillBatch* p);
+// ---- prompt prefill (prefill.cpp, prefill_engine.hip) ----
+// A session's prefill buffers: tokens ids[0..n) at positions pos0 .. pos0 + n
+// - 1 through every layer, up to kPfMaxRows positions a pass, on the session's
+// KV cache; writes the KV rows, no logits. create returns nullptr (error set)
+// when the shape does not fit. run queues on the session's stream `st` and does
+// not wait: ids (pinned) must stay as they are until it has.
+struct PrefillEngine;
+PrefillEngine* prefill_engine_create(const xp_session* s);
+int prefill_engine_run(PrefillEngine* p, const uint32_t* ids, uint32_t n, uint32_t pos0, hipStream_t st);
+void prefill_engine_destroy(PrefillEngine* p);
+constexpr uint32_t kPfMaxRows = 2048;
+struct PfPrepArgs {
+    float* x;                  // [rows_pad][K] residual stream
+    const float* y;            // [ysplit][rows_pad][K] sublayer output, k splits (mode 1)
+    uint32_t ysplit;
+    const float* w_post;
+    const float* w_pre;
+    void* a;                   // staged operand
+    float* asum;
+    uint32_t K, rows, rows_pad;   // rows_pad: rows rounded up to whole 16-row tiles
+    bool wide;                 // 32-row operand tiles (the 128-row GEMM), not 16
+    float eps;
+    const uint32_t* tok;       // non-null: x is set to the embedding of tok[row] (mode 0)
+    const void* ewq;
+    const void* esc;
+    const float* etable;
+    uint32_t vocab;
+    int efmt;
+    float escale;
+};
+int launch_pf_prep(const PfPrepArgs& a, hipStream_t st);
+struct PfGemmPlan {
+    int shape;                 // 0, 1: the small kernel with two or four row tiles; 2: 128-row tiles
+    uint32_t m_wgs, n_tiles, splits, qsplit;
+};
+PfGemmPlan plan_pf_gemm(uint32_t rows, uint32_t cols, uint32_t nblk, bool geglu, int n_cu);
+struct PfGemmArgs {
+    const void* a;
+    const float* asum;
+    MvMatDesc mats[3];         // concatenated columns, or gate and up (out unused)
+    uint32_t n_mats, nblk, m_tiles;
+    float* out;                // [splits][16 m_tiles][ldo]
+    uint32_t ldo;
+    void* a_out;               // GeGLU: the staged operand of the next GEMM
+    float* asum_out;
+    uint32_t nblk_out;
+    uint32_t tile0[3];         // set by launch_pf_gemm, as the following
+    uint32_t m_wgs, n_tiles, splits, qsplit;
+};
+int launch_pf_gemm(PfGemmArgs a, const PfGemmPlan& p, int fmt, bool geglu, hipStream_t st, const char* who);
+struct PfQkArgs {
+    const float* qkv;          // [splits][rows_pad][(n_heads + 2 kv_heads) 256]
+    uint32_t splits, rows, rows_pad, n_heads, kv_heads, pos0;
+    const float* qw;
+    const float* kw;
+    float eps;
+    uint16_t* kc;              // fp16 caches [t][kv_heads][256]
+    uint16_t* vc;
+    _Float16* qh;              // [kv_heads][rows][group][256] fp16 terms of q 2^e
+    _Float16* ql;
+    float* qscale;             // [kv_heads][rows][group] 2^-e
+};
+int launch_pf_qk(const PfQkArgs& a, float theta, hipStream_t st);
+constexpr uint32_t kPfRecord = 260;   // floats of a key split's record per query row: max, sum, 2 unused, 256 values
+struct PfAttnArgs {
+    const _Float16* qh;
+    const _Float16* ql;
+    const float* qscale;
+    const uint16_t* kc;
+    const uint16_t* vc;
+    uint32_t rows, kv_heads, pos0, window;   // window 0: every earlier key
+    float scale;
+    void* a;                   // staged o operand, nblk blocks of k
+    float* asum;
+    uint32_t nblk;
+    bool wide;
+    float* part;               // [kv_heads][row workgroups][splits][32][kPfRecord], splits > 1
+};
+uint32_t pf_attn_splits(uint32_t rows, uint32_t group, uint32_t kv_heads, uint32_t max_keys, int n_cu);
+int launch_pf_attn(const PfAttnArgs& a, uint32_t group, uint32_t splits, hipStream_t st);
 // The session's host draw and Philox uniform (decode.cpp:1873-1917).
 uint32_t draw(float* val, uint32_t* idx, uint32_t n, float temperature, uint32_t top_k,
               float top_p, double u);
