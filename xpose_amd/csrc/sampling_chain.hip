@@ -5,18 +5,13 @@
 // that decode does not call; here each is one gfx950 kernel behind an
 // xp_<name> entry point with the reference's argument meaning.
 //
-// Every kernel evaluates what the reference evaluates in the same order:
-// chain p is walked k = p, p + nparts, ... by one thread (consecutive threads
-// take consecutive chains, so each step of the walk is one coalesced load
-// across the wave), and the serial finalisers stay serial. Sums, comparisons,
-// the division and the cumulative walks are therefore bit-identical to the
-// reference's fp32 arithmetic on the same inputs; only exp (the device libm
-// against llvmpipe's) can differ in the last bits.
-//
-// Where the reference's one-thread-per-chain form would hold a 64-entry array
-// per thread (topk_partial), the array lives in LDS, column-major across the
-// workgroup's threads so that a step of the insertion touches 64 different
-// banks. rank selection stages the candidate list through LDS in tiles.
+// Every kernel evaluates what the reference evaluates in the same order where
+// the order shows: a chain's sum is added in chain order, the serial
+// finalisers stay serial. Sums, comparisons, the division and the cumulative
+// walks are therefore bit-identical to the reference's fp32 arithmetic on the
+// same inputs; only exp (the device libm against llvmpipe's) can differ in the
+// last bits. What has no order (exponentials, maxima, the choice of the best k)
+// is spread over as many threads as the chip has.
 #include "xp_device.hpp"
 #include "xp_launch.hpp"
 
@@ -30,7 +25,10 @@ constexpr uint32_t kTopkThreads = 64;      // one wave: 64 x 64 x 8 B = 32 KiB o
 constexpr uint32_t kRankTile = 2048;       // candidates staged per LDS tile
 constexpr uint32_t kNone = 0xFFFFFFFFu;    // unfilled candidate slot
 
-uint32_t blocks(uint32_t n, uint32_t per) { return (n + per - 1) / per; }
+uint32_t blocks(uint32_t n, uint32_t per) { return (n - 1u) / per + 1u; }   // n > 0
+
+// topk_partial: a wave a chain or a thread a chain.
+bool topk_by_wave(uint32_t n, uint32_t nparts) { return n / nparts >= 16u || nparts <= 4096u; }
 
 }  // namespace
 
@@ -39,13 +37,40 @@ __global__ __launch_bounds__(kScThreads) void temperature_kernel(float* x, float
     if (i < n) x[i] = x[i] * inv_temp;
 }
 
+// Chains share a workgroup sixteen at a time: thread t takes chain t % 16 and
+// rows t / 16, t / 16 + 16, ... (element p + row * nparts), so a wave's load is
+// four 64-byte runs and a chain's elements are worked on by sixteen threads.
+// With a thread a chain (a few thousand threads, one load in flight each)
+// n = 262144 in 4096 chains took 8.6 us for the maximum and 14.8 for the
+// exponentials; now 2.6 and 3.7.
+constexpr uint32_t kChainW = 16;                         // chains a workgroup
+constexpr uint32_t kChainR = kScThreads / kChainW;       // rows at a time
+constexpr uint32_t kChainU = 4;                          // rows in flight a thread
+
+// The maximum is the same in any order.
 __global__ __launch_bounds__(kScThreads) void reduce_max_partial_kernel(float* pmax, const float* x,
                                                                         uint32_t n, uint32_t nparts) {
-    const uint32_t p = blockIdx.x * kScThreads + threadIdx.x;
-    if (p >= nparts) return;
+    __shared__ float sm[kChainR][kChainW];
+    const uint32_t c = threadIdx.x % kChainW, r0 = threadIdx.x / kChainW, p = blockIdx.x * kChainW + c;
     float m = -INFINITY;
-    for (uint32_t k = p; k < n; k += nparts) m = fmaxf(m, x[k]);
-    pmax[p] = m;
+    if (p < nparts)
+        for (uint64_t k = p + uint64_t(r0) * nparts; k < n; k += uint64_t(kChainU * kChainR) * nparts) {
+            float v[kChainU];
+#pragma unroll
+            for (uint32_t u = 0; u < kChainU; ++u) {
+                const uint64_t e = k + uint64_t(u * kChainR) * nparts;
+                v[u] = e < n ? x[e] : -INFINITY;
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < kChainU; ++u) m = fmaxf(m, v[u]);
+        }
+    sm[r0][c] = m;
+    __syncthreads();
+    if (r0 == 0 && p < nparts) {
+#pragma unroll
+        for (uint32_t r = 1; r < kChainR; ++r) m = fmaxf(m, sm[r][c]);
+        pmax[p] = m;
+    }
 }
 
 // The maximum is the same in any order (fmax drops NaNs either way), so the
@@ -64,20 +89,48 @@ __global__ __launch_bounds__(1024) void reduce_max_final_kernel(float* stats, co
     }
 }
 
+// The exponentials of a 64-row tile by all threads, then each chain's sum in
+// chain order by one. `out` may alias `x`: every element is read and written
+// by the same thread, its tile's loads before its stores.
 __global__ __launch_bounds__(kScThreads) void softmax_exp_partial_kernel(float* out, float* psum,
                                                                          const float* x,
                                                                          const float* stats,
                                                                          uint32_t n, uint32_t nparts) {
-    const uint32_t p = blockIdx.x * kScThreads + threadIdx.x;
-    if (p >= nparts) return;
+    constexpr uint32_t TR = kChainU * kChainR;
+    __shared__ float se[TR][kChainW + 1];
+    const uint32_t c = threadIdx.x % kChainW, r0 = threadIdx.x / kChainW, p = blockIdx.x * kChainW + c;
+    const bool live = p < nparts;
     const float m = stats[0];
+    const uint64_t rows = (uint64_t(n) + nparts - 1u) / nparts;   // of the longest chain
     float s = 0.0f;
-    for (uint32_t k = p; k < n; k += nparts) {
-        const float e = expf(x[k] - m);
-        out[k] = e;
-        s += e;
+    for (uint64_t t = 0; t < rows; t += TR) {
+        float v[kChainU];
+#pragma unroll
+        for (uint32_t u = 0; u < kChainU; ++u) {
+            const uint64_t e = p + (t + r0 + u * kChainR) * nparts;
+            v[u] = live && e < n ? x[e] : 0.0f;
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < kChainU; ++u) {
+            const uint64_t e = p + (t + r0 + u * kChainR) * nparts;
+            const float g = expf(v[u] - m);
+            if (live && e < n) out[e] = g;
+            se[r0 + u * kChainR][c] = g;
+        }
+        __syncthreads();
+        if (r0 == 0 && live && p < n) {
+            const uint64_t mine = (uint64_t(n) - p + nparts - 1u) / nparts;   // this chain's rows
+            const uint32_t left = uint32_t(mine > t ? (mine - t < TR ? mine - t : TR) : 0u);
+            if (left == TR) {
+#pragma unroll
+                for (uint32_t r = 0; r < TR; ++r) s += se[r][c];
+            } else {
+                for (uint32_t r = 0; r < left; ++r) s += se[r][c];
+            }
+        }
+        __syncthreads();
     }
-    psum[p] = s;
+    if (r0 == 0 && live) psum[p] = s;
 }
 
 __global__ __launch_bounds__(kScThreads) void reduce_sum_partial_kernel(float* out, const float* in,
@@ -89,21 +142,46 @@ __global__ __launch_bounds__(kScThreads) void reduce_sum_partial_kernel(float* o
     out[p] = s;
 }
 
-// Serial, as the reference: the fp32 sum depends on its order. The loads are
-// issued 16 ahead; the adds stay in order.
-__global__ void reduce_sum_final_kernel(float* stats, const float* psum, uint32_t nparts) {
-    if (threadIdx.x != 0) return;
-    float s = 0.0f;
-    uint32_t p = 0;
-    for (; p + 16 <= nparts; p += 16) {
-        float v[16];
+// Serial, as the reference: the fp32 sum depends on its order. All threads
+// bring a tile to LDS (zeros past the end: cum + 0 is cum) and one wave adds,
+// every lane the same, sixteen words read ahead of their adds: one dependent
+// add every 8 cycles is what is left (4096 sums: 64 -> 15 us; loads issued
+// sixteen at a time from memory waited out a round trip each time).
+constexpr uint32_t kSerTile = 4096;
+__device__ __forceinline__ uint32_t serial_tile(float* tile, const float* src, uint32_t base, uint32_t n) {
+    const uint32_t m = min(kSerTile, n - base);
+    for (uint32_t i = threadIdx.x; i < (m + 31u) / 32u * 32u; i += kScThreads) tile[i] = i < m ? src[base + i] : 0.0f;
+    __syncthreads();
+    return m;
+}
+__device__ __forceinline__ void ld16(float (&v)[16], const float* p) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) v[i] = psum[p + i];
-#pragma unroll
-        for (int i = 0; i < 16; ++i) s += v[i];
+    for (int i = 0; i < 4; ++i) {
+        const float4 q = *reinterpret_cast<const float4*>(p + 4 * i);
+        v[4 * i] = q.x; v[4 * i + 1] = q.y; v[4 * i + 2] = q.z; v[4 * i + 3] = q.w;
     }
-    for (; p < nparts; ++p) s += psum[p];
-    stats[1] = s;
+}
+
+__global__ __launch_bounds__(kScThreads) void reduce_sum_final_kernel(float* stats, const float* psum, uint32_t nparts) {
+    __shared__ __attribute__((aligned(16))) float tile[kSerTile + 32];
+    float s = 0.0f;
+    for (uint32_t base = 0; base < nparts; base += kSerTile) {
+        __syncthreads();
+        const uint32_t m = serial_tile(tile, psum, base, nparts);
+        if (threadIdx.x < kWave) {
+            float v[16], w[16];
+            ld16(v, tile);
+            for (uint32_t i = 0; i < m; i += 32) {
+                ld16(w, tile + i + 16u);
+#pragma unroll
+                for (int j = 0; j < 16; ++j) s += v[j];
+                ld16(v, tile + i + 32u);                 // the tile has the words to spare
+#pragma unroll
+                for (int j = 0; j < 16; ++j) s += w[j];
+            }
+        }
+    }
+    if (threadIdx.x == 0) stats[1] = s;
 }
 
 __global__ __launch_bounds__(kScThreads) void softmax_normalize_kernel(float* out, const float* stats,
@@ -143,6 +221,236 @@ __global__ __launch_bounds__(kTopkThreads) void topk_partial_kernel(float* cval,
     for (uint32_t j = 0; j < k; ++j) {
         cval[size_t(p) * k + j] = bv[j][t];
         cidx[size_t(p) * k + j] = bi[j][t];
+    }
+}
+
+// ---- exact best k (<= 64) of a wave's values --------------------------------
+// Values live in registers, R a lane, with an order-preserving key (0 = no
+// candidate) and an id; the best k by (value desc, id asc) are found without
+// sorting: the k-th largest key bit by bit from the top, each bit one count
+// over the wave (R compares and ballots), starting below the bits that the
+// largest and the smallest lane maximum share (at least 64 keys reach the
+// latter) and ending as soon as a cut keeps exactly k; only a tie across the
+// cut is resolved further, by id. A thread inserting element by element into
+// its own sorted list in LDS took 5.1 ms for 256 chains of 1024 and k = 64,
+// this 11.7 us.
+__device__ __forceinline__ uint32_t order_key(float v) {
+    const uint32_t u = __float_as_uint(v);
+    return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+}
+__device__ __forceinline__ uint32_t value_key(float v) { return order_key(v + 0.0f); }   // -0 ties with 0
+
+template <int R>
+__device__ __forceinline__ uint32_t count_ge(const uint32_t (&key)[R], uint32_t t) {
+    uint32_t c = 0;
+#pragma unroll
+    for (int j = 0; j < R; ++j) c += uint32_t(__popcll(__ballot(key[j] >= t)));
+    return c;
+}
+__device__ __forceinline__ uint32_t lanes_below(unsigned long long m) {
+    return __builtin_amdgcn_mbcnt_hi(uint32_t(m >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(m), 0u));
+}
+// LDS written by some lanes of a wave is read by others of it: in order in
+// the hardware, kept in order in the code.
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// The survivors (at most k, in no order) to sv / si; returns their number.
+template <int R>
+__device__ __forceinline__ uint32_t wave_best(const float (&v)[R], const uint32_t (&id)[R],
+                                              const uint32_t (&key)[R], uint32_t k, float* sv, uint32_t* si) {
+    uint32_t t = 1u, cnt = count_ge(key, 1u), tie_id = kNone;
+    bool ties = false;
+    if (cnt > k) {
+        uint32_t lm = 0;
+#pragma unroll
+        for (int j = 0; j < R; ++j) lm = max(lm, key[j]);
+        uint32_t hi = lm, lo = lm;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            hi = max(hi, uint32_t(__shfl_xor(int(hi), o, kWave)));
+            lo = min(lo, uint32_t(__shfl_xor(int(lo), o, kWave)));
+        }
+        hi = __builtin_amdgcn_readfirstlane(hi);
+        lo = __builtin_amdgcn_readfirstlane(lo);
+        const int nb = hi == lo ? 0 : 32 - __builtin_clz(hi ^ lo);
+        t = nb >= 32 ? 0u : hi & ~((1u << nb) - 1u);
+        cnt = t == 0u ? 0xFFFFFFFFu : count_ge(key, t);
+        for (int b = nb - 1; b >= 0 && cnt != k; --b) {
+            const uint32_t c = count_ge(key, t | (1u << b));
+            if (c >= k) {
+                t |= 1u << b;
+                cnt = c;
+            }
+        }
+        if (cnt > k) {   // the k-th largest key is t, with more of it than fit
+            ties = true;
+            uint32_t g = 0;
+#pragma unroll
+            for (int j = 0; j < R; ++j) g += uint32_t(__popcll(__ballot(key[j] > t)));
+            tie_id = 0u;
+            for (int b = 31; b >= 0; --b) {
+                const uint32_t u = tie_id | ((1u << b) - 1u);
+                uint32_t c = 0;
+#pragma unroll
+                for (int j = 0; j < R; ++j) c += uint32_t(__popcll(__ballot(key[j] == t && id[j] <= u)));
+                if (c < k - g) tie_id |= 1u << b;
+            }
+        }
+    }
+    uint32_t m = 0;
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+        const bool take = ties ? key[j] > t : key[j] >= t;
+        const unsigned long long b = __ballot(take);
+        const uint32_t at = m + lanes_below(b);
+        if (take) {
+            sv[at] = v[j];
+            si[at] = id[j];
+        }
+        m += uint32_t(__popcll(b));
+    }
+    if (ties) {
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+            const bool take = key[j] == t && id[j] <= tie_id;
+            const unsigned long long b = __ballot(take);
+            const uint32_t at = m + lanes_below(b);
+            if (take && at < k) {
+                sv[at] = v[j];
+                si[at] = id[j];
+            }
+            m = min(k, m + uint32_t(__popcll(b)));
+        }
+    }
+    wave_lds_sync();
+    return m;
+}
+
+// Lane i < m of a wave's m survivors: its value, id and rank, the number of
+// survivors that beat it.
+__device__ __forceinline__ uint32_t wave_rank(const float* sv, const uint32_t* si, uint32_t m, float& v, uint32_t& d) {
+    const uint32_t lane = threadIdx.x % kWave, i = min(lane, m - 1u);
+    v = sv[i];
+    d = si[i];
+    uint32_t rank = 0;
+    for (uint32_t j = 0; j < m; ++j) {
+        const float w = sv[j];
+        const uint32_t e = si[j];
+        rank += (w > v) | ((w == v) & (e < d));
+    }
+    return rank;
+}
+
+constexpr int kBestR = 17;                               // the survivors so far, and 16 new values a lane
+
+// Chain p's best k (descending, the earliest index first among equals),
+// unfilled slots (-inf, none): one wave a chain, 1024 elements at a time.
+__global__ __launch_bounds__(kWave) void topk_partial_wave_kernel(float* cval, uint32_t* cidx, const float* x,
+                                                                 uint32_t n, uint32_t nparts, uint32_t k) {
+    __shared__ float sv[kTopkMax];
+    __shared__ uint32_t si[kTopkMax];
+    const uint32_t p = blockIdx.x, lane = threadIdx.x;
+    uint32_t m = 0;
+    for (uint64_t r0 = 0; p + r0 * nparts < n; r0 += 1024u) {
+        float v[kBestR];
+        uint32_t id[kBestR], key[kBestR];
+        v[0] = lane < m ? sv[lane] : 0.0f;
+        id[0] = lane < m ? si[lane] : kNone;
+        key[0] = lane < m ? value_key(v[0]) : 0u;
+#pragma unroll
+        for (int j = 1; j < kBestR; ++j) {
+            const uint64_t e = p + (r0 + uint32_t(j - 1) * kWave + lane) * nparts;
+            id[j] = uint32_t(e);
+            v[j] = e < n ? x[e] : -INFINITY;
+        }
+#pragma unroll
+        for (int j = 1; j < kBestR; ++j) key[j] = v[j] > -INFINITY ? value_key(v[j]) : 0u;   // no NaN either
+        wave_lds_sync();                                 // slot 0 is read before it is written
+        m = wave_best(v, id, key, k, sv, si);
+    }
+    float v = -INFINITY;
+    uint32_t d = kNone, rank = lane;
+    if (m > 0) {
+        float wv;
+        uint32_t wd;
+        const uint32_t wr = wave_rank(sv, si, m, wv, wd);
+        if (lane < m) {
+            v = wv;
+            d = wd;
+            rank = wr;
+        }
+    }
+    if (rank < k) {                                      // lanes past m fill the slots past the survivors
+        cval[size_t(p) * k + rank] = v;
+        cidx[size_t(p) * k + rank] = d;
+    }
+}
+
+// The best k <= 64 of a candidate list by (value desc, index asc) to oval /
+// oidx[rank], one workgroup: each wave keeps the best k of its share, the
+// first wave the best of those. Slots with no candidate of that rank are not
+// written. Counting every candidate against every other took 512 us for 16384; this
+// takes 17.
+__global__ __launch_bounds__(1024) void topk_rank_wave_kernel(float* oval, uint32_t* oidx, const float* cval,
+                                                             const uint32_t* cidx, uint32_t ncand, uint32_t k) {
+    __shared__ float sv[16][kTopkMax];
+    __shared__ uint32_t si[16][kTopkMax];
+    __shared__ uint32_t sm[16];
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+    const uint32_t waves = blockDim.x / kWave;
+    uint32_t m = 0;
+    for (uint64_t b = uint64_t(wave) * 1024u; b < ncand; b += uint64_t(waves) * 1024u) {
+        float v[kBestR];
+        uint32_t id[kBestR], key[kBestR];
+        v[0] = lane < m ? sv[wave][lane] : 0.0f;
+        id[0] = lane < m ? si[wave][lane] : kNone;
+        key[0] = lane < m ? value_key(v[0]) : 0u;
+#pragma unroll
+        for (int j = 1; j < kBestR; ++j) {
+            const uint64_t i = b + uint32_t(j - 1) * kWave + lane;
+            v[j] = i < ncand ? cval[i] : 0.0f;
+            id[j] = i < ncand ? cidx[i] : kNone;
+        }
+#pragma unroll
+        for (int j = 1; j < kBestR; ++j) {
+            if (id[j] != kNone && v[j] != v[j]) {        // beaten by none and beating none: rank 0, as ever
+                oval[0] = v[j];
+                oidx[0] = id[j];
+            }
+            key[j] = id[j] != kNone && v[j] == v[j] ? value_key(v[j]) : 0u;
+        }
+        wave_lds_sync();
+        m = wave_best(v, id, key, k, sv[wave], si[wave]);
+    }
+    if (waves > 1) {
+        if (lane == 0) sm[wave] = m;
+        __syncthreads();
+        if (wave != 0) return;
+        float v[kBestR];
+        uint32_t id[kBestR], key[kBestR];
+        v[0] = 0.0f;
+        id[0] = kNone;
+        key[0] = 0u;
+#pragma unroll
+        for (int j = 1; j < kBestR; ++j) {
+            const bool in = uint32_t(j - 1) < waves && lane < sm[j - 1];
+            v[j] = in ? sv[j - 1][lane] : 0.0f;
+            id[j] = in ? si[j - 1][lane] : kNone;
+            key[j] = in ? value_key(v[j]) : 0u;
+        }
+        wave_lds_sync();
+        m = wave_best(v, id, key, k, sv[0], si[0]);
+    }
+    if (wave != 0 || m == 0) return;
+    float v;
+    uint32_t d;
+    const uint32_t rank = wave_rank(sv[0], si[0], m, v, d);
+    if (lane < m) {
+        oval[rank] = v;
+        oidx[rank] = d;
     }
 }
 
@@ -192,58 +500,166 @@ __global__ __launch_bounds__(kScThreads) void topk_mask_kernel(float* logits, co
     if (logits[i] < t) logits[i] = -INFINITY;
 }
 
-// One thread, serial over k (the reference's top-p is a single work-item).
-__global__ void topp_cutoff_kernel(float* w, uint32_t k, float p) {
-    if (threadIdx.x != 0) return;
+// Serial over k (the reference's top-p is a single work-item): a wave brings
+// 256 weights at a time to LDS (zeros past the end) and every lane adds them in
+// order, sixteen read at once.
+constexpr uint32_t kDrawTile = 256;
+__device__ __forceinline__ float lane_f(float v, uint32_t l) {
+    return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), int(l)));
+}
+__device__ __forceinline__ void draw_tile(float* tile, const float* w, uint32_t b, uint32_t k) {
+    wave_lds_sync();
+#pragma unroll
+    for (uint32_t j = 0; j < kDrawTile; j += kWave)
+        tile[j + threadIdx.x] = b + j + threadIdx.x < k ? w[b + j + threadIdx.x] : 0.0f;
+    wave_lds_sync();
+}
+__device__ __forceinline__ float serial_total(float* tile, const float* w, uint32_t k) {
     float total = 0.0f;
-    for (uint32_t j = 0; j < k; ++j) total += w[j];
-    if (!(total > 0.0f)) return;
-    float cum = 0.0f;
-    for (uint32_t j = 0; j < k; ++j) {
-        if (cum >= p * total) w[j] = 0.0f;
-        else cum += w[j];
+    for (uint32_t b = 0; b < k; b += kDrawTile) {
+        draw_tile(tile, w, b, k);
+        for (uint32_t i = 0; i < kDrawTile && b + i < k; i += 16) {
+            float v[16];
+            ld16(v, tile + i);
+#pragma unroll
+            for (int j = 0; j < 16; ++j) total += v[j];
+        }
     }
+    return total;
 }
 
-__global__ void multinomial_sample_kernel(float* out, uint32_t* idx_out, const float* w,
-                                          const uint32_t* idx, uint32_t k, float u) {
-    if (threadIdx.x != 0) return;
-    float total = 0.0f;
-    for (uint32_t j = 0; j < k; ++j) total += w[j];
-    const float target = u * total;
+__global__ __launch_bounds__(kWave) void topp_cutoff_kernel(float* w, uint32_t k, float p) {
+    __shared__ __attribute__((aligned(16))) float tile[kDrawTile];
+    const float total = serial_total(tile, w, k);
+    if (!(total > 0.0f)) return;
+    // every weight from the first whose running mass before it reaches the
+    // cut on: past it the mass no longer grows
+    const float cut = p * total;
     float cum = 0.0f;
-    uint32_t chosen = 0u;
-    float cw = 0.0f;
-    for (uint32_t j = 0; j < k; ++j) {
-        cum += w[j];
-        if (w[j] > 0.0f) { chosen = idx[j]; cw = w[j]; }
-        if (cum > target) break;
+    uint32_t keep = kNone;
+    for (uint32_t b = 0; b < k && keep == kNone; b += kDrawTile) {
+        draw_tile(tile, w, b, k);
+        for (uint32_t i = 0; i < kDrawTile && b + i < k && keep == kNone; i += 16) {
+            float v[16];
+            ld16(v, tile + i);
+#pragma unroll
+            for (int j = 0; j < 16; ++j) {
+                if (keep == kNone && cum >= cut) keep = b + i + j;
+                cum += v[j];
+            }
+        }
     }
+    if (keep == kNone) return;
+    for (uint64_t j = uint64_t(keep) + threadIdx.x; j < k; j += kWave) w[j] = 0.0f;
+}
+
+__global__ __launch_bounds__(kWave) void multinomial_sample_kernel(float* out, uint32_t* idx_out, const float* w,
+                                                                   const uint32_t* idx, uint32_t k, float u) {
+    __shared__ __attribute__((aligned(16))) float tile[kDrawTile];
+    const float target = u * serial_total(tile, w, k);
+    float cum = 0.0f, cw = 0.0f;
+    uint32_t at = kNone;                                 // the last weight above zero up to the stop
+    bool stop = false;
+    for (uint32_t b = 0; b < k && !stop; b += kDrawTile) {
+        draw_tile(tile, w, b, k);
+        for (uint32_t i = 0; i < kDrawTile && b + i < k && !stop; i += 16) {
+            float v[16];
+            ld16(v, tile + i);
+#pragma unroll
+            for (int j = 0; j < 16; ++j) {
+                if (!stop && v[j] > 0.0f) {
+                    at = b + i + j;
+                    cw = v[j];
+                }
+                cum += v[j];
+                stop = stop || cum > target;
+            }
+        }
+    }
+    if (threadIdx.x != 0) return;
+    const uint32_t chosen = at == kNone ? 0u : idx[at];
     out[0] = float(chosen);
     out[1] = cw;
     idx_out[0] = chosen;
 }
 
-__global__ void multinomial_strided_kernel(float* out, uint32_t* idx_out, const float* w,
-                                           const float* psum, const float* stats, uint32_t n,
-                                           uint32_t nparts, float u) {
-    if (threadIdx.x != 0) return;
+// The chain whose running mass passes the target, then the element in it: the
+// sums and their order are the reference's, from LDS tiles as in
+// reduce_sum_final (4096 chains: 250 -> 32 us; one thread loaded as it
+// went). Sixteen running sums are formed before their largest is held
+// against the target; only then is the first that passes looked for.
+__global__ __launch_bounds__(kScThreads) void multinomial_strided_kernel(float* out, uint32_t* idx_out, const float* w,
+                                                                         const float* psum, const float* stats,
+                                                                         uint32_t n, uint32_t nparts, float u) {
+    __shared__ __attribute__((aligned(16))) float tile[kSerTile + 32];
+    __shared__ uint32_t found;
     const float target = u * stats[1];
     float cum = 0.0f;
-    uint32_t chain = nparts - 1u;
-    for (uint32_t p = 0; p < nparts; ++p) {
-        const float s = psum[p];
-        if (cum + s > target) { chain = p; break; }
-        cum += s;
+    uint32_t chain = kNone;
+    if (threadIdx.x == 0) found = 0u;
+    for (uint32_t base = 0; base < nparts; base += kSerTile) {
+        __syncthreads();
+        if (found) break;
+        const uint32_t m = serial_tile(tile, psum, base, nparts);
+        if (threadIdx.x < kWave) {
+            // sixteen running sums; true once one has passed the target
+            auto step = [&](const float (&v)[16], uint32_t at) {
+                float c[16];
+                c[0] = cum + v[0];
+#pragma unroll
+                for (int j = 1; j < 16; ++j) c[j] = c[j - 1] + v[j];
+                float mx = c[0];
+#pragma unroll
+                for (int j = 1; j < 16; ++j) mx = fmaxf(mx, c[j]);
+                if (!(mx > target)) {
+                    cum = c[15];
+                    return false;
+                }
+                uint32_t f = 0;
+#pragma unroll
+                for (int j = 15; j >= 0; --j)
+                    if (c[j] > target) f = uint32_t(j);
+                // the running sum is not added past the chosen chain
+#pragma unroll
+                for (int j = 0; j < 15; ++j)
+                    if (f == uint32_t(j) + 1u) cum = c[j];
+                chain = base + at + f;
+                return true;
+            };
+            float v[16], x[16];
+            ld16(v, tile);
+            for (uint32_t i = 0; i < m; i += 32) {
+                ld16(x, tile + i + 16u);
+                if (step(v, i)) break;
+                ld16(v, tile + i + 32u);
+                if (step(x, i + 16u)) break;
+            }
+            if (threadIdx.x == 0 && chain != kNone) found = 1u;
+        }
     }
+    if (threadIdx.x >= kWave) return;
+    if (chain == kNone) chain = nparts - 1u;
     uint32_t chosen = chain;
-    for (uint32_t e = chain; e < n; e += nparts) {
-        chosen = e;
-        cum += w[e];
-        if (cum > target) break;
+    float cw = 0.0f;
+    bool stop = false;
+    for (uint64_t b = chain; b < n && !stop; b += uint64_t(kWave) * nparts) {
+        const uint64_t e = b + uint64_t(threadIdx.x) * nparts;
+        const float v = e < n ? w[e] : 0.0f;
+        const uint64_t left = (uint64_t(n) - b + nparts - 1u) / nparts;
+        const uint32_t m = uint32_t(left < kWave ? left : kWave);
+        for (uint32_t j = 0; j < m; ++j) {
+            chosen = uint32_t(b + uint64_t(j) * nparts);
+            cw = lane_f(v, j);
+            cum += cw;
+            if (cum > target) {
+                stop = true;
+                break;
+            }
+        }
     }
+    if (threadIdx.x != 0) return;
     out[0] = float(chosen);
-    out[1] = w[chosen];
+    out[1] = cw;
     idx_out[0] = chosen;
 }
 
@@ -263,11 +679,6 @@ constexpr uint32_t kSelKeep = 256;           // survivors ranked (k + ties)
 static_assert(kTopkMax <= kSelKeep, "the ranked output fits the survivors' slots");
 constexpr uint32_t kSelCopies = 16;          // histogram copies
 constexpr uint32_t kSelStride = kSelCopies + 1u;   // words per bin (padded: the sum reads bins apart)
-
-__device__ __forceinline__ uint32_t order_key(float v) {
-    const uint32_t u = __float_as_uint(v);
-    return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-}
 
 __global__ __launch_bounds__(kSelThreads) void select_rows_kernel(float* oval, uint32_t* oidx,
                                                                   const float* cval,
@@ -556,7 +967,7 @@ int xp_reduce_max_partial(float* pmax, const float* x, uint32_t n, uint32_t npar
                           xp_stream stream) {
     XP_REQUIRE(pmax && x, "null pointer");
     XP_REQUIRE(n > 0 && nparts > 0, "n and nparts must be positive");
-    hipLaunchKernelGGL(reduce_max_partial_kernel, dim3(blocks(nparts, kScThreads)), dim3(kScThreads),
+    hipLaunchKernelGGL(reduce_max_partial_kernel, dim3(blocks(nparts, kChainW)), dim3(kScThreads),
                        0, as_stream(stream), pmax, x, n, nparts);
     XP_SC_LAUNCH("xp_reduce_max_partial");
 }
@@ -573,7 +984,7 @@ int xp_softmax_exp_partial(float* out, float* psum, const float* x, const float*
                            uint32_t nparts, xp_stream stream) {
     XP_REQUIRE(out && psum && x && stats, "null pointer");
     XP_REQUIRE(n > 0 && nparts > 0, "n and nparts must be positive");
-    hipLaunchKernelGGL(softmax_exp_partial_kernel, dim3(blocks(nparts, kScThreads)), dim3(kScThreads),
+    hipLaunchKernelGGL(softmax_exp_partial_kernel, dim3(blocks(nparts, kChainW)), dim3(kScThreads),
                        0, as_stream(stream), out, psum, x, stats, n, nparts);
     XP_SC_LAUNCH("xp_softmax_exp_partial");
 }
@@ -590,7 +1001,7 @@ int xp_reduce_sum_partial(float* out, const float* in, uint32_t n, uint32_t npar
 int xp_reduce_sum_final(float* stats, const float* psum, uint32_t nparts, xp_stream stream) {
     XP_REQUIRE(stats && psum, "null pointer");
     XP_REQUIRE(nparts > 0, "nparts must be positive");
-    hipLaunchKernelGGL(reduce_sum_final_kernel, dim3(1), dim3(64), 0, as_stream(stream), stats, psum,
+    hipLaunchKernelGGL(reduce_sum_final_kernel, dim3(1), dim3(kScThreads), 0, as_stream(stream), stats, psum,
                        nparts);
     XP_SC_LAUNCH("xp_reduce_sum_final");
 }
@@ -608,8 +1019,14 @@ int xp_topk_partial(float* cval, uint32_t* cidx, const float* x, uint32_t n, uin
     XP_REQUIRE(cval && cidx && x, "null pointer");
     XP_REQUIRE(n > 0 && nparts > 0, "n and nparts must be positive");
     XP_REQUIRE(k >= 1 && k <= kTopkMax, "k=%u must be in [1, %u]", k, kTopkMax);
-    hipLaunchKernelGGL(topk_partial_kernel, dim3(blocks(nparts, kTopkThreads)), dim3(kTopkThreads), 0,
-                       as_stream(stream), cval, cidx, x, n, nparts, k);
+    // a wave a chain, unless the chains are short and so many that a thread
+    // each fills the chip
+    if (topk_by_wave(n, nparts))
+        hipLaunchKernelGGL(topk_partial_wave_kernel, dim3(nparts), dim3(kWave), 0, as_stream(stream), cval, cidx, x,
+                           n, nparts, k);
+    else
+        hipLaunchKernelGGL(topk_partial_kernel, dim3(blocks(nparts, kTopkThreads)), dim3(kTopkThreads), 0,
+                           as_stream(stream), cval, cidx, x, n, nparts, k);
     XP_SC_LAUNCH("xp_topk_partial");
 }
 
@@ -617,8 +1034,12 @@ int xp_topk_rank_select(float* oval, uint32_t* oidx, const float* cval, const ui
                         uint32_t ncand, uint32_t k, xp_stream stream) {
     XP_REQUIRE(oval && oidx && cval && cidx, "null pointer");
     XP_REQUIRE(ncand > 0 && k > 0, "ncand and k must be positive");
-    hipLaunchKernelGGL(topk_rank_select_kernel, dim3(blocks(ncand, kScThreads)), dim3(kScThreads), 0,
-                       as_stream(stream), oval, oidx, cval, cidx, ncand, k);
+    if (k <= kTopkMax)
+        hipLaunchKernelGGL(topk_rank_wave_kernel, dim3(1), dim3(kWave * std::min(16u, blocks(ncand, 1024u))), 0,
+                           as_stream(stream), oval, oidx, cval, cidx, ncand, k);
+    else
+        hipLaunchKernelGGL(topk_rank_select_kernel, dim3(blocks(ncand, kScThreads)), dim3(kScThreads), 0,
+                           as_stream(stream), oval, oidx, cval, cidx, ncand, k);
     XP_SC_LAUNCH("xp_topk_rank_select");
 }
 
@@ -651,7 +1072,7 @@ int xp_multinomial_strided(float* out, uint32_t* idx_out, const float* w, const 
                            xp_stream stream) {
     XP_REQUIRE(out && idx_out && w && psum && stats, "null pointer");
     XP_REQUIRE(n > 0 && nparts > 0 && nparts <= n, "need 0 < nparts <= n");
-    hipLaunchKernelGGL(multinomial_strided_kernel, dim3(1), dim3(64), 0, as_stream(stream), out,
+    hipLaunchKernelGGL(multinomial_strided_kernel, dim3(1), dim3(kScThreads), 0, as_stream(stream), out,
                        idx_out, w, psum, stats, n, nparts, u);
     XP_SC_LAUNCH("xp_multinomial_strided");
 }
