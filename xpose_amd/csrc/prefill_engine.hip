@@ -626,8 +626,9 @@ __global__ __launch_bounds__(256) void pf_qk_kernel(PfQkArgs a, RopeFreq f) {
 // into LDS in that key order while it is staged (8 keys x 8 dims a thread).
 // q and p are two fp16 terms each (22 bits), K and V fp16 as the cache holds
 // them, sums fp32. Two waves a SIMD (a lone wave issues a vector instruction
-// every 8 cycles), cache rows through raw buffers (a scalar offset a tile, no
-// address arithmetic; rows past the last key read as zeros).
+// every 8 cycles), cache rows through raw buffers, one descriptor a load that
+// starts at the load's first row (scalar arithmetic only) and ends at the last
+// key: rows past it read as zeros.
 constexpr uint32_t kPaThreads = 512, kPaKeys = 128;
 constexpr float kPaPScale = 16384.0f;   // p 2^14: the low term keeps bits to 2^-38
 
@@ -666,7 +667,11 @@ __global__ __launch_bounds__(kPaThreads) void pf_attn_kernel(PfAttnArgs a) {
         kn = min(kn, k0 + per * kPaKeys);
     }
     const uint32_t rowb = a.kv_heads * 512u;                           // bytes between cache rows
-    const rsrc_t rk = make_rsrc(a.kc, (last + 1u) * rowb), rv = make_rsrc(a.vc, (last + 1u) * rowb);
+    const uint32_t kvbytes = (last + 1u) * rowb;
+    auto rows_from = [&](const uint16_t* base, uint32_t row) {
+        const uint32_t off = __builtin_amdgcn_readfirstlane(min(row * rowb, kvbytes));
+        return make_rsrc(reinterpret_cast<const unsigned char*>(base) + off, __builtin_amdgcn_readfirstlane(kvbytes - off));
+    };
     // K: 16-byte word i of the tile = key i / 32, word i % 32. V: thread's key
     // chunk tid / 32 = (32-key step, group) and dims 8 (tid % 32) ..
     const uint32_t ko = (tid / 32u) * rowb + kvh * 512u + (tid % 32u) * 16u;
@@ -676,10 +681,10 @@ __global__ __launch_bounds__(kPaThreads) void pf_attn_kernel(PfAttnArgs a) {
     auto load = [&](uint32_t kt) {
 #pragma unroll
         for (uint32_t r = 0; r < 8; ++r)
-            kr[r] = __builtin_amdgcn_raw_buffer_load_b128(rk, int(ko), int((kt + 16u * r) * rowb), 0);
+            kr[r] = __builtin_amdgcn_raw_buffer_load_b128(rows_from(a.kc, kt + 16u * r), int(ko), 0, 0);
 #pragma unroll
         for (uint32_t j = 0; j < 8; ++j)
-            vr[j] = __builtin_amdgcn_raw_buffer_load_b128(rv, int(vo), int((kt + (j & 3u) + (j >> 2) * 16u) * rowb), 0);
+            vr[j] = __builtin_amdgcn_raw_buffer_load_b128(rows_from(a.vc, kt + (j & 3u) + (j >> 2) * 16u), int(vo), 0, 0);
     };
     auto store = [&]() {
 #pragma unroll
