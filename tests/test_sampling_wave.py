@@ -145,3 +145,49 @@ def test_gpu_topp_and_draw_any_k(xp, xo, k):
             X.call("xp_multinomial_sample", do.vp, di.vp, dw.vp, dids.vp, k, u, None)
             X.synchronize()
             assert int(di.download(np.uint32)[0]) == int(oi[0]) and np.array_equal(do.download(np.float32), out)
+
+
+def terms(kind, n, seed):
+    r = np.random.default_rng(seed)
+    if kind == "even":                        # a softmax's chain sums
+        return r.uniform(0.5, 1.5, n).astype(np.float32)
+    if kind == "wide":
+        return np.exp(r.normal(0, 6, n)).astype(np.float32)
+    if kind == "ties":                        # whole numbers and halves of the sum's last place, on both sides of even
+        return np.concatenate([np.float32([2.0 ** 23 + 1]), r.integers(0, 6, n).astype(np.float32) / 2])[:n]
+    if kind == "tiny":                        # denormal terms and sums
+        return (r.integers(0, 1 << 22, n).astype(np.uint32)).view(np.float32)
+    x = np.where(r.random(n) < 0.8, 0.0, r.random(n)).astype(np.float32)
+    if kind == "signs":
+        x -= np.float32(0.05)
+        x[::7] = -0.0
+    elif kind == "inf":
+        x[n // 2] = np.inf
+    elif kind == "nan":
+        x[2 * n // 3] = np.nan
+    return x
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["even", "wide", "ties", "tiny", "sparse", "signs", "inf", "nan"])
+@pytest.mark.parametrize("n", [1, 63, 64, 257, 4096, 4100, 9000])
+def test_gpu_serial_sums_bit_exact(xp, xo, kind, n):
+    """The sums and the place in them, which are formed in blocks, against the
+    oracle's one chain of adds."""
+    X, L = xp, xo.lib()
+    print(f"case serial sums {kind} n={n}", flush=True)
+    w = terms(kind, n, n)
+    dw, ds = dbuf(X, w), dbuf(X, np.zeros(2, np.float32))
+    X.call("xp_reduce_sum_final", ds.vp, dw.vp, n, None)
+    X.synchronize()
+    want = np.zeros(2, np.float32)
+    L.xo_reduce_sum_final(want, w, n)
+    assert np.array_equal(ds.download(np.float32), want, equal_nan=True)
+    do, di = X.DeviceBuffer(8), X.DeviceBuffer(4)
+    for u in (0.0, 0.013, 0.24, 0.5000001, 0.77, 0.9999, 1.0, 1.01, -1.0):
+        X.call("xp_multinomial_strided", do.vp, di.vp, dw.vp, dw.vp, ds.vp, n, n, u, None)
+        X.synchronize()
+        out, oi = np.empty(2, np.float32), np.empty(1, np.uint32)
+        L.xo_multinomial_strided(out, oi, w, w, want, n, n, np.float32(u))
+        assert int(di.download(np.uint32)[0]) == int(oi[0]), u
+        assert np.array_equal(do.download(np.float32), out, equal_nan=True), u

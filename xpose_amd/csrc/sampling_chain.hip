@@ -142,15 +142,68 @@ __global__ __launch_bounds__(kScThreads) void reduce_sum_partial_kernel(float* o
     out[p] = s;
 }
 
-// Serial, as the reference: the fp32 sum depends on its order. All threads
-// bring a tile to LDS (zeros past the end: cum + 0 is cum) and one wave adds,
-// every lane the same, sixteen words read ahead of their adds: one dependent
-// add every 8 cycles is what is left (4096 sums: 64 -> 15 us; loads issued
-// sixteen at a time from memory waited out a round trip each time).
-constexpr uint32_t kSerTile = 4096;
+// ---- serial sums ------------------------------------------------------------
+// The reference adds in one order, and the fp32 sum depends on it. A lone chain
+// of dependent adds costs 8 cycles each (15 us for 4096), but where the running
+// sum s keeps its exponent, adding v >= 0 adds the whole number rint(v / u) of
+// s's last places u, whatever the terms before it: only a tie (v / u halfway
+// between two whole numbers) looks at s, at its last bit. So a wave adds a
+// block at once, as whole numbers below 2^24, and gets the serial sum bit for bit.
+// A block in which the exponent would change, or with a term that is negative,
+// not finite or more than a quarter of s, is refused and added one by one.
+__device__ __forceinline__ bool sum_scale(float s, int& sh) {
+    const uint32_t e = __float_as_uint(s) >> 23;
+    sh = 150 - int(e);                                   // v / u = v 2^sh
+    return e - 1u < 254u;                                // positive, normal, finite
+}
+// s + the last places `more`, if that keeps the exponent.
+__device__ __forceinline__ bool sum_grow(float& s, float more, uint32_t ties) {
+    const uint32_t b = __float_as_uint(s);
+    if (!(more + float(ties) < 8388608.0f - float(b & 0x7FFFFFu))) return false;
+    s = __uint_as_float(b + uint32_t(more) + ties);
+    return true;
+}
+// 256 terms, four a lane in any order; ties are refused.
+__device__ __forceinline__ bool sum_block4(float& s, float4 v) {
+    int sh;
+    if (!sum_scale(s, sh)) return false;
+    const float t[4] = {v.x, v.y, v.z, v.w};
+    bool ok = true;
+    float q = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float r = __builtin_amdgcn_ldexpf(t[i], sh), k = __builtin_rintf(r);
+        ok = ok && r >= 0.0f && r < 4194304.0f && fabsf(r - k) != 0.5f;
+        q += k;                                          // exact: at most 2^24
+    }
+    if (__ballot(!ok) != 0ull) return false;
+    return sum_grow(s, wave_sum(q), 0u);                 // a sum past 2^24 may round, but not to below it
+}
+// 64 terms, one a lane in order.
+__device__ __forceinline__ bool sum_block(float& s, float v) {
+    int sh;
+    if (!sum_scale(s, sh)) return false;
+    const float r = __builtin_amdgcn_ldexpf(v, sh), w = floorf(r), f = r - w;
+    if (__ballot(!(r >= 0.0f && r < 4194304.0f)) != 0ull) return false;
+    const float k = w + (f > 0.5f ? 1.0f : 0.0f);
+    unsigned long long tie = __ballot(f == 0.5f);
+    uint32_t up = 0;
+    if (tie != 0ull) {
+        const unsigned long long odd = __ballot((uint32_t(k) & 1u) != 0u);
+        for (; tie != 0ull; tie &= tie - 1u) {           // to even: up where the sum before it, and its whole part, are odd
+            const int i = __builtin_ctzll(tie);
+            up += (__float_as_uint(s) + uint32_t(__builtin_popcountll(odd & ((2ull << i) - 1ull))) + up) & 1u;
+        }
+    }
+    return sum_grow(s, wave_sum(k), up);
+}
+
+constexpr uint32_t kSerTile = 4096, kSerBlock = 256;
+static_assert(kSerTile % kSerBlock == 0, "whole blocks");
+// A tile of terms to LDS by all threads, zeros up to a whole block (s + 0 is s).
 __device__ __forceinline__ uint32_t serial_tile(float* tile, const float* src, uint32_t base, uint32_t n) {
     const uint32_t m = min(kSerTile, n - base);
-    for (uint32_t i = threadIdx.x; i < (m + 31u) / 32u * 32u; i += kScThreads) tile[i] = i < m ? src[base + i] : 0.0f;
+    for (uint32_t i = threadIdx.x; i < (m + kSerBlock - 1u) / kSerBlock * kSerBlock; i += kScThreads) tile[i] = i < m ? src[base + i] : 0.0f;
     __syncthreads();
     return m;
 }
@@ -162,22 +215,26 @@ __device__ __forceinline__ void ld16(float (&v)[16], const float* p) {
     }
 }
 
+// 4096 sums: 64 us by one thread from memory, 18.6 as a chain of adds from
+// LDS, 16.1 in blocks.
 __global__ __launch_bounds__(kScThreads) void reduce_sum_final_kernel(float* stats, const float* psum, uint32_t nparts) {
-    __shared__ __attribute__((aligned(16))) float tile[kSerTile + 32];
+    __shared__ __attribute__((aligned(16))) float tile[kSerTile];
     float s = 0.0f;
     for (uint32_t base = 0; base < nparts; base += kSerTile) {
         __syncthreads();
         const uint32_t m = serial_tile(tile, psum, base, nparts);
         if (threadIdx.x < kWave) {
-            float v[16], w[16];
-            ld16(v, tile);
-            for (uint32_t i = 0; i < m; i += 32) {
-                ld16(w, tile + i + 16u);
+            for (uint32_t i = 0; i < m; i += kSerBlock) {
+                if (sum_block4(s, *reinterpret_cast<const float4*>(tile + i + 4u * threadIdx.x))) continue;
+                for (uint32_t j = i; j < i + kSerBlock; j += kWave) {
+                    if (sum_block(s, tile[j + threadIdx.x])) continue;
+                    for (uint32_t h = j; h < j + kWave; h += 16) {
+                        float v[16];
+                        ld16(v, tile + h);
 #pragma unroll
-                for (int j = 0; j < 16; ++j) s += v[j];
-                ld16(v, tile + i + 32u);                 // the tile has the words to spare
-#pragma unroll
-                for (int j = 0; j < 16; ++j) s += w[j];
+                        for (int x = 0; x < 16; ++x) s += v[x];
+                    }
+                }
             }
         }
     }
@@ -584,14 +641,15 @@ __global__ __launch_bounds__(kWave) void multinomial_sample_kernel(float* out, u
 }
 
 // The chain whose running mass passes the target, then the element in it: the
-// sums and their order are the reference's, from LDS tiles as in
-// reduce_sum_final (4096 chains: 250 -> 32 us; one thread loaded as it
-// went). Sixteen running sums are formed before their largest is held
-// against the target; only then is the first that passes looked for.
+// sums and their order are the reference's, from LDS tiles in blocks as in
+// reduce_sum_final (4096 chains: 250 us by one thread, 31.5 as a chain of adds,
+// 20.8 so). A block added at once has no negative term: it is passed over where
+// its end has not passed the target. In one that may hold the place, sixteen
+// running sums are formed before their largest is held against the target.
 __global__ __launch_bounds__(kScThreads) void multinomial_strided_kernel(float* out, uint32_t* idx_out, const float* w,
                                                                          const float* psum, const float* stats,
                                                                          uint32_t n, uint32_t nparts, float u) {
-    __shared__ __attribute__((aligned(16))) float tile[kSerTile + 32];
+    __shared__ __attribute__((aligned(16))) float tile[kSerTile];
     __shared__ uint32_t found;
     const float target = u * stats[1];
     float cum = 0.0f;
@@ -626,13 +684,24 @@ __global__ __launch_bounds__(kScThreads) void multinomial_strided_kernel(float* 
                 chain = base + at + f;
                 return true;
             };
-            float v[16], x[16];
-            ld16(v, tile);
-            for (uint32_t i = 0; i < m; i += 32) {
-                ld16(x, tile + i + 16u);
-                if (step(v, i)) break;
-                ld16(v, tile + i + 32u);
-                if (step(x, i + 16u)) break;
+            for (uint32_t i = 0; i < m && chain == kNone; i += kSerBlock) {
+                float c = cum;
+                if (sum_block4(c, *reinterpret_cast<const float4*>(tile + i + 4u * threadIdx.x)) && !(c > target)) {
+                    cum = c;
+                    continue;
+                }
+                for (uint32_t j = i; j < i + kSerBlock && chain == kNone; j += kWave) {
+                    c = cum;
+                    if (sum_block(c, tile[j + threadIdx.x]) && !(c > target)) {
+                        cum = c;
+                        continue;
+                    }
+                    for (uint32_t h = j; h < j + kWave; h += 16) {
+                        float v[16];
+                        ld16(v, tile + h);
+                        if (step(v, h)) break;
+                    }
+                }
             }
             if (threadIdx.x == 0 && chain != kNone) found = 1u;
         }
