@@ -290,7 +290,7 @@ __global__ __launch_bounds__(kTopkThreads) void topk_partial_kernel(float* cval,
 // latter) and ending as soon as a cut keeps exactly k; only a tie across the
 // cut is resolved further, by id. A thread inserting element by element into
 // its own sorted list in LDS took 5.1 ms for 256 chains of 1024 and k = 64,
-// this 11.7 us.
+// this 11 us.
 __device__ __forceinline__ uint32_t order_key(float v) {
     const uint32_t u = __float_as_uint(v);
     return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
@@ -314,34 +314,28 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_wave_barrier();
 }
 
-// The survivors (at most k, in no order) to sv / si; returns their number.
+// Bits b and below of the k-th largest key, from the top, into t: until the
+// cut keeps at most `enough`. cnt keys reach t.
 template <int R>
-__device__ __forceinline__ uint32_t wave_best(const float (&v)[R], const uint32_t (&id)[R],
-                                              const uint32_t (&key)[R], uint32_t k, float* sv, uint32_t* si) {
-    uint32_t t = 1u, cnt = count_ge(key, 1u), tie_id = kNone;
+__device__ __forceinline__ int search_cut(const uint32_t (&key)[R], uint32_t k, uint32_t enough, int b, uint32_t& t, uint32_t& cnt) {
+    for (; b >= 0 && cnt > enough; --b) {
+        const uint32_t c = count_ge(key, t | (1u << b));
+        if (c >= k) {
+            t |= 1u << b;
+            cnt = c;
+        }
+    }
+    return b;
+}
+// The survivors (at most k, in no order) to sv / si; returns their number.
+// cnt keys reach t, which has the k-th largest key's bits above b.
+template <int R>
+__device__ __forceinline__ uint32_t wave_cut(const float (&v)[R], const uint32_t (&id)[R], const uint32_t (&key)[R],
+                                             uint32_t k, int bit, uint32_t t, uint32_t cnt, float* sv, uint32_t* si) {
+    uint32_t tie_id = kNone;
     bool ties = false;
     if (cnt > k) {
-        uint32_t lm = 0;
-#pragma unroll
-        for (int j = 0; j < R; ++j) lm = max(lm, key[j]);
-        uint32_t hi = lm, lo = lm;
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            hi = max(hi, uint32_t(__shfl_xor(int(hi), o, kWave)));
-            lo = min(lo, uint32_t(__shfl_xor(int(lo), o, kWave)));
-        }
-        hi = __builtin_amdgcn_readfirstlane(hi);
-        lo = __builtin_amdgcn_readfirstlane(lo);
-        const int nb = hi == lo ? 0 : 32 - __builtin_clz(hi ^ lo);
-        t = nb >= 32 ? 0u : hi & ~((1u << nb) - 1u);
-        cnt = t == 0u ? 0xFFFFFFFFu : count_ge(key, t);
-        for (int b = nb - 1; b >= 0 && cnt != k; --b) {
-            const uint32_t c = count_ge(key, t | (1u << b));
-            if (c >= k) {
-                t |= 1u << b;
-                cnt = c;
-            }
-        }
+        search_cut(key, k, k, bit, t, cnt);
         if (cnt > k) {   // the k-th largest key is t, with more of it than fit
             ties = true;
             uint32_t g = 0;
@@ -386,17 +380,86 @@ __device__ __forceinline__ uint32_t wave_best(const float (&v)[R], const uint32_
     return m;
 }
 
+// A search over 17 registers a lane is 51 instructions a bit: once the cut
+// keeps kBestFew, those move to LDS and back to five registers a lane.
+constexpr int kFewR = 5;
+constexpr uint32_t kBestFew = kFewR * kWave;
+struct BestFew {
+    float v[kBestFew];
+    uint32_t id[kBestFew];
+};
+template <int R>
+__device__ __forceinline__ uint32_t wave_best(const float (&v)[R], const uint32_t (&id)[R], const uint32_t (&key)[R],
+                                              uint32_t k, BestFew& few, float* sv, uint32_t* si) {
+    uint32_t t = 1u, cnt = count_ge(key, 1u);
+    int bit = -1;
+    if (cnt > k) {
+        uint32_t lm = 0;
+#pragma unroll
+        for (int j = 0; j < R; ++j) lm = max(lm, key[j]);
+        uint32_t hi = lm, lo = lm;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            hi = max(hi, uint32_t(__shfl_xor(int(hi), o, kWave)));
+            lo = min(lo, uint32_t(__shfl_xor(int(lo), o, kWave)));
+        }
+        hi = __builtin_amdgcn_readfirstlane(hi);
+        lo = __builtin_amdgcn_readfirstlane(lo);
+        const int nb = hi == lo ? 0 : 32 - __builtin_clz(hi ^ lo);
+        t = nb >= 32 ? 0u : hi & ~((1u << nb) - 1u);
+        cnt = t == 0u ? 0xFFFFFFFFu : count_ge(key, t);
+        bit = search_cut(key, k, max(k, kBestFew), nb - 1, t, cnt);
+    }
+    if (cnt > kBestFew) return wave_cut(v, id, key, k, bit, t, cnt, sv, si);   // that many equal keys
+    uint32_t m = 0;
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+        const bool take = key[j] >= t;
+        const unsigned long long b = __ballot(take);
+        const uint32_t at = m + lanes_below(b);
+        if (take) {
+            few.v[at] = v[j];
+            few.id[at] = id[j];
+        }
+        m += uint32_t(__popcll(b));
+    }
+    wave_lds_sync();
+    const uint32_t lane = threadIdx.x % kWave;
+    float fv[kFewR];
+    uint32_t fid[kFewR], fkey[kFewR];
+#pragma unroll
+    for (int j = 0; j < kFewR; ++j) {
+        const uint32_t at = uint32_t(j) * kWave + lane;
+        fv[j] = few.v[at];
+        fid[j] = at < m ? few.id[at] : kNone;
+        fkey[j] = at < m ? value_key(fv[j]) : 0u;
+    }
+    wave_lds_sync();
+    return wave_cut(fv, fid, fkey, k, bit, t, cnt, sv, si);
+}
+
 // Lane i < m of a wave's m survivors: its value, id and rank, the number of
-// survivors that beat it.
-__device__ __forceinline__ uint32_t wave_rank(const float* sv, const uint32_t* si, uint32_t m, float& v, uint32_t& d) {
-    const uint32_t lane = threadIdx.x % kWave, i = min(lane, m - 1u);
-    v = sv[i];
-    d = si[i];
+// survivors that beat it. The slots past m are filled with what beats nothing.
+__device__ __forceinline__ uint32_t wave_rank(float* sv, uint32_t* si, uint32_t m, float& v, uint32_t& d) {
+    const uint32_t lane = threadIdx.x % kWave;
+    if (lane >= m) {
+        sv[lane] = -INFINITY;
+        si[lane] = kNone;
+    }
+    wave_lds_sync();
+    v = sv[lane];
+    d = si[lane];
     uint32_t rank = 0;
-    for (uint32_t j = 0; j < m; ++j) {
-        const float w = sv[j];
-        const uint32_t e = si[j];
-        rank += (w > v) | ((w == v) & (e < d));
+    for (uint32_t j = 0; j < m; j += 8) {
+        float w[8];
+        uint32_t e[8];
+#pragma unroll
+        for (uint32_t i = 0; i < 8; ++i) {
+            w[i] = sv[j + i];
+            e[i] = si[j + i];
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < 8; ++i) rank += (w[i] > v) | ((w[i] == v) & (e[i] < d));
     }
     return rank;
 }
@@ -407,8 +470,9 @@ constexpr int kBestR = 17;                               // the survivors so far
 // unfilled slots (-inf, none): one wave a chain, 1024 elements at a time.
 __global__ __launch_bounds__(kWave) void topk_partial_wave_kernel(float* cval, uint32_t* cidx, const float* x,
                                                                  uint32_t n, uint32_t nparts, uint32_t k) {
-    __shared__ float sv[kTopkMax];
-    __shared__ uint32_t si[kTopkMax];
+    __shared__ __attribute__((aligned(16))) float sv[kTopkMax];
+    __shared__ __attribute__((aligned(16))) uint32_t si[kTopkMax];
+    __shared__ BestFew few;
     const uint32_t p = blockIdx.x, lane = threadIdx.x;
     uint32_t m = 0;
     for (uint64_t r0 = 0; p + r0 * nparts < n; r0 += 1024u) {
@@ -426,7 +490,7 @@ __global__ __launch_bounds__(kWave) void topk_partial_wave_kernel(float* cval, u
 #pragma unroll
         for (int j = 1; j < kBestR; ++j) key[j] = v[j] > -INFINITY ? value_key(v[j]) : 0u;   // no NaN either
         wave_lds_sync();                                 // slot 0 is read before it is written
-        m = wave_best(v, id, key, k, sv, si);
+        m = wave_best(v, id, key, k, few, sv, si);
     }
     float v = -INFINITY;
     uint32_t d = kNone, rank = lane;
@@ -450,11 +514,12 @@ __global__ __launch_bounds__(kWave) void topk_partial_wave_kernel(float* cval, u
 // oidx[rank], one workgroup: each wave keeps the best k of its share, the
 // first wave the best of those. Slots with no candidate of that rank are not
 // written. Counting every candidate against every other took 512 us for 16384; this
-// takes 17.
+// takes 14.5 (17 where every bit was a count over all registers).
 __global__ __launch_bounds__(1024) void topk_rank_wave_kernel(float* oval, uint32_t* oidx, const float* cval,
                                                              const uint32_t* cidx, uint32_t ncand, uint32_t k) {
-    __shared__ float sv[16][kTopkMax];
-    __shared__ uint32_t si[16][kTopkMax];
+    __shared__ __attribute__((aligned(16))) float sv[16][kTopkMax];
+    __shared__ __attribute__((aligned(16))) uint32_t si[16][kTopkMax];
+    __shared__ BestFew few[16];
     __shared__ uint32_t sm[16];
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
     const uint32_t waves = blockDim.x / kWave;
@@ -480,7 +545,7 @@ __global__ __launch_bounds__(1024) void topk_rank_wave_kernel(float* oval, uint3
             key[j] = id[j] != kNone && v[j] == v[j] ? value_key(v[j]) : 0u;
         }
         wave_lds_sync();
-        m = wave_best(v, id, key, k, sv[wave], si[wave]);
+        m = wave_best(v, id, key, k, few[wave], sv[wave], si[wave]);
     }
     if (waves > 1) {
         if (lane == 0) sm[wave] = m;
@@ -499,7 +564,7 @@ __global__ __launch_bounds__(1024) void topk_rank_wave_kernel(float* oval, uint3
             key[j] = in ? value_key(v[j]) : 0u;
         }
         wave_lds_sync();
-        m = wave_best(v, id, key, k, sv[0], si[0]);
+        m = wave_best(v, id, key, k, few[0], sv[0], si[0]);
     }
     if (wave != 0 || m == 0) return;
     float v;
