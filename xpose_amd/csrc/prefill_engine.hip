@@ -65,8 +65,9 @@ __device__ __forceinline__ void pf_stage(u32x4* A, float* asum, bool wide, uint3
 // ---- residual add, norms and operand staging -------------------------------
 // W waves a row (thread i of them takes the row's 8-element words i, i + 64 W,
 // ...), RW rows a workgroup. Many rows: one wave a row, so every reduction
-// stays in the wave, and 16 rows a workgroup, which writes whole operand
-// lines. Few rows: enough waves that a thread holds one word and has every
+// stays in the wave, and 8 rows a workgroup, which writes whole 128-byte
+// operand lines (16 left half of the CUs without one at 2000 rows: 15.0 us,
+// 8: 12.5). Few rows: enough waves that a thread holds one word and has every
 // split's share of it in flight at once.
 //   tok set: x = embedding of tok[row]; stage rmsnorm(x) (1 + w_pre)
 //   else:    x += rmsnorm(sum of the y splits) (1 + w_post), staged likewise
@@ -889,7 +890,7 @@ int launch_pf_prep(const PfPrepArgs& a, hipStream_t st) {
     hipLaunchKernelGGL((pf_prep_kernel<NC, RW, W>), dim3((a.rows_pad + RW - 1u) / RW), dim3(RW * W * kWave), 0, st, a)
     if (a.K <= 1536u) {
         if (a.rows_pad <= 256u) XP_PREP(1, 1, 3);
-        else XP_PREP(3, 16, 1);
+        else XP_PREP(3, 8, 1);
     } else {
         XP_PREP(1, 1, 16);
     }
