@@ -137,9 +137,10 @@ __global__ __launch_bounds__(kPfThreads, 4) void attention_scores_prefill_kernel
     const uint32_t c32 = lane % 32u, half = lane / 32u;
     const size_t rows = size_t(group) * n_query;          // of this kv head
     const size_t kst = size_t(kv_heads) * head_dim;
-    for (uint32_t t0 = blockIdx.y * kAsKeys; t0 < seq_len; t0 += gridDim.y * kAsKeys)
+    for (uint64_t tb = uint64_t(blockIdx.y) * kAsKeys; tb < seq_len; tb += uint64_t(gridDim.y) * kAsKeys)
     for (uint32_t kvh = blockIdx.z; kvh < kv_heads; kvh += gridDim.z)
     for (size_t r0 = size_t(blockIdx.x) * kAsRows; r0 < rows; r0 += size_t(gridDim.x) * kAsRows) {
+        const uint32_t t0 = uint32_t(tb);
         // the positions of the tile's queries: one run, or two where it
         // crosses from one head to the next (then any position)
         const uint32_t nr = uint32_t(rows - r0 < kAsRows ? rows - r0 : kAsRows);
