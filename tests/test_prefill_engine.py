@@ -64,3 +64,66 @@ def test_gpu_prefill_engine_equals_token_steps(xp, shape, tokens, start, fmt):
         err = np.abs(x - y).max(axis=1)
         assert np.all(err <= 1e-3 * np.abs(y).max(axis=1)), (i, int(err.argmax()), err.max())
     assert np.abs(la - lb).max() <= 1e-3 * np.abs(lb).max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,tokens,start,window,cached,ahead", [
+    # rows the workgroup's later rows no longer see, near and far ends of its 32 positions
+    ("gemma", 40, 700, 512, (189, 195), ()), ("mha", 65, 600, 512, (90, 119), ()),
+    ("narrow", 33, 40, 20, (25, 38), ()), ("mha", 40, 40, 1, (39,), ()),
+    # rows ahead: the last of a tile of positions, the first of one, the keys of a split span
+    ("gemma", 40, 0, 512, (), (7, 30)), ("mha", 130, 0, 512, (), (31, 128)), ("narrow", 70, 3000, 0, (), (17, 64)),
+    ("gemma", 200, 3000, 0, (), (60, 197)), ("mha", 40, 40, 1, (39,), (20,))])
+def test_gpu_prefill_engine_non_finite_values(xp, shape, tokens, start, window, cached, ahead):
+    """A value row that is not finite reaches the positions that see it and no
+    other: rows already cached that leave a window inside the prompt, and rows
+    of the prompt itself whose values pass float16's largest, ahead of others.
+    Layer 1's KV rows show layer 0's attention: XP_PREFILL_TOKENS (a token step
+    reads its own span only) gives those of the positions that see none."""
+    X = xp
+    print(f"case prefill engine not finite {shape} tokens={tokens} start={start} window={window}", flush=True)
+    bad_tok = 5
+    got = {}
+    for pm in (X.XP_PREFILL_AUTO, X.XP_PREFILL_TOKENS):
+        cfg = X.XpConfig.gemma3_1b(n_layers=2, vocab=1024, global_every=2 if window else 0, max_seq=max(512, start + tokens),
+                                   sliding_window=window or 512, prefill_mode=pm, **SHAPES[shape])
+        kvd = cfg.n_kv_heads * cfg.head_dim
+        sess = X.DecodeSession(cfg)
+        sess.synthesize(3)
+        emb = np.random.default_rng(7).normal(0, 1, (cfg.vocab, cfg.hidden)).astype(np.float32)
+        emb[bad_tok] = 0.0
+        emb[bad_tok, 0] = 1.0                # its normed row: sqrt(hidden) in one place
+        sess.upload(-1, X.T_EMBED, emb)
+        if ahead:
+            # that place's weight block scaled so that its nibbles of -8 overflow
+            # (8 s sqrt(hidden) = 72 000), other tokens' values (32 nibbles of
+            # about 4.6 s) far from it
+            sc = X.synth_tensor(cfg, 3, 0, X.T_V | X.T_SCALES).view(np.float16).copy()
+            sc[:4 * kvd:4] = 9000.0 / np.sqrt(cfg.hidden)
+            sess.upload(0, X.T_V | X.T_SCALES, sc)
+            sess.upload(0, X.T_ATTN_NORM, np.zeros(cfg.hidden, np.float32))
+        for l in range(2):
+            for which in (0, 1):
+                if start:
+                    rows = X.synth_normal_f16(start * kvd, 5, 2 * l + which).reshape(start, kvd)
+                    for i, p in enumerate(cached):
+                        if l == 0 and which == 1:
+                            rows[p, i::16] = np.float16([np.inf, np.nan][i % 2]).view(np.uint16)
+                    sess.kv_upload(l, which, 0, rows)
+        sess.set_position(start)
+        ids = np.random.default_rng(tokens).integers(6, cfg.vocab, tokens).astype(np.uint32)
+        ids[list(ahead)] = bad_tok
+        sess.prefill(ids)
+        v0 = sess.kv_download(0, 1, start, tokens).view(np.float16).reshape(tokens, kvd)
+        got[pm] = [sess.kv_download(1, w, start, tokens).view(np.float16).astype(np.float64).reshape(tokens, kvd) for w in (0, 1)]
+        sess.close()
+        bad = np.array(sorted(set(cached) | {start + i for i in np.flatnonzero(~np.isfinite(v0).all(1))}))
+        assert set(bad) == set(cached) | {start + i for i in ahead}
+    pos = np.arange(start, start + tokens)[:, None]
+    sees = ((bad <= pos) & ((bad + window > pos) if window else True)).any(1)
+    assert not sees.all()
+    for a, b in zip(got[X.XP_PREFILL_AUTO], got[X.XP_PREFILL_TOKENS]):
+        assert np.isfinite(b[~sees]).all()
+        assert np.array_equal(np.isfinite(a).all(1)[:-1], ~sees[:-1])   # the last token takes a token step
+        err = np.abs(a[~sees] - b[~sees]).max(axis=1)
+        assert np.all(err <= 1e-3 * np.abs(b[~sees]).max(axis=1)), (int(err.argmax()), err.max())
