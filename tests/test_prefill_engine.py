@@ -9,6 +9,9 @@ against the oracle (activations as two bf16 terms, 2^-18; cache rows fp16,
 workgroups with one row more and one less, prompts that end in a partly filled
 tile, one that takes two chunks, spans split over workgroups, one to four
 query heads a KV head, the sliding window's edge, both scale formats."""
+import ctypes as C
+import os
+
 import numpy as np
 import pytest
 
@@ -127,3 +130,53 @@ def test_gpu_prefill_engine_non_finite_values(xp, shape, tokens, start, window, 
         assert np.array_equal(np.isfinite(a).all(1)[:-1], ~sees[:-1])   # the last token takes a token step
         err = np.abs(a[~sees] - b[~sees]).max(axis=1)
         assert np.all(err <= 1e-3 * np.abs(b[~sees]).max(axis=1)), (int(err.argmax()), err.max())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,start,window,qscale,splits", [
+    (32, 0, 0, 1.0, 2), (200, 1000, 0, 1.0, 5), (200, 1000, 512, 1.0, 2), (500, 0, 512, 1.5, 2), (300, 1500, 0, 1.5, 4)])
+def test_gpu_prefill_engine_attention_error(xp, rows, start, window, qscale, splits):
+    """The engine's attention by itself, from the row records it writes before
+    they are staged, against float64 of the same queries and cache: no further
+    off than xp_attention_decode, the token steps' attention, is on the same
+    rows. Both are measured here, so the bar needs no constant but 5 % for the
+    rows drawn (float32 sums in another order; 0.93 to 1.01 of it measured)."""
+    X = xp
+    print(f"case prefill attention error rows={rows} start={start} window={window}", flush=True)
+    lib = C.CDLL(os.path.join(os.path.dirname(__file__), "native", "prefill_attention.so"))
+    rec, G, D, n = lib.test_prefill_attention_record(), 4, 256, start + rows
+    r = np.random.default_rng(rows + start)
+    k, v = (r.normal(0, 1, (n, D)).astype(np.float16) for _ in range(2))
+    q = (r.normal(0, qscale, (rows, G, D))).astype(np.float32)
+    e = 13 - np.floor(np.log2(np.abs(q).max(-1, keepdims=True)))
+    qq = q * np.exp2(e).astype(np.float32)
+    qh = qq.astype(np.float16)
+    ql = (qq - qh.astype(np.float32)).astype(np.float16)
+    wgs = -(-rows * G // 32)
+    buf = {m: X.DeviceBuffer.from_array(a) for m, a in dict(qh=qh, ql=ql, qs=np.exp2(-e).astype(np.float32), k=k, v=v, q=q).items()}
+    pad = -(-rows // 32) * 32
+    part, a, asum, out = (X.DeviceBuffer(4 * m) for m in (wgs * splits * 32 * rec, pad * G * D, pad * G * D // 32, G * D))
+    f = C.c_float
+    rc = lib.test_prefill_attention(buf["qh"].vp, buf["ql"].vp, buf["qs"].vp, buf["k"].vp, buf["v"].vp, rows, 1, G, start,
+                                    window, f(0.0625), a.vp, asum.vp, part.vp, splits)
+    assert rc == 0
+    X.synchronize()
+    p = part.download(np.float32).astype(np.float64).reshape(wgs, splits, 32, rec)
+    w = np.exp2(p[..., 0] - p[..., 0].max(1, keepdims=True))       # record: max (of score log2(e)), sum, 2 unused, row
+    got = ((w[..., None] * p[..., 4:]).sum(1) / (w * p[..., 1]).sum(1)[..., None]).reshape(-1, G, D)[:rows]
+    step = np.empty((rows, G, D), np.float32)
+    for i in range(rows):
+        span = min(start + i + 1, window) if window else start + i + 1
+        X.call("xp_attention_decode", out.vp, C.c_void_p(buf["q"].ptr + 4 * i * G * D), buf["k"].vp, buf["v"].vp, G, 1, D, span,
+               start + i + 1 - span, f(0.0625), None)
+        X.synchronize()
+        step[i] = out.download(np.float32).reshape(G, D)
+    s = (q.reshape(-1, D).astype(np.float64) @ k.astype(np.float64).T / 16).reshape(rows, G, n)
+    t, pos = np.arange(n)[None], np.arange(start, n)[:, None]
+    off = (t > pos) | ((t + window <= pos) if window else False)
+    s = np.where(off[:, None], -np.inf, s)
+    s = np.exp(s - s.max(-1, keepdims=True))
+    want = ((s / s.sum(-1, keepdims=True)).reshape(-1, n) @ v.astype(np.float64)).reshape(rows, G, D)
+    err, bar = (np.linalg.norm(x - want) / np.linalg.norm(want) for x in (got, step))
+    print(f"engine {err:.3e} step {bar:.3e}", flush=True)
+    assert err <= 1.05 * bar

@@ -97,10 +97,28 @@ def build_oracle(verbose: bool = False) -> str:
     return ORACLE_LIB
 
 
+NATIVE_DIR = os.path.join(ROOT, "tests", "native")
+
+
+def build_test_helpers(verbose: bool = False) -> None:
+    """The tests' host-side helpers over libxpose.so's internals: a shared
+    object beside each tests/native/*.cpp."""
+    for f in sorted(os.listdir(NATIVE_DIR)):
+        if not f.endswith(".cpp"):
+            continue
+        src = os.path.join(NATIVE_DIR, f)
+        out = src[:-4] + ".so"
+        _run([HIPCC, "-O1", "-fPIC", "-std=c++17", "-Wall", "-shared", src, "-o", out + ".tmp", "-L",
+              os.path.dirname(LIB), "-l:libxpose.so", "-Wl,-rpath,$ORIGIN/../../xpose_amd"], verbose)
+        os.replace(out + ".tmp", out)
+
+
 def build_all(verbose: bool = False) -> None:
     build_oracle(verbose)
     build_lib(verbose)
     build_cli(verbose)
+    if os.path.isdir(NATIVE_DIR):
+        build_test_helpers(verbose)
 
 
 if __name__ == "__main__":

@@ -625,8 +625,16 @@ __global__ __launch_bounds__(256) void pf_qk_kernel(PfQkArgs a, RopeFreq f) {
 // (4 g + 0..3, 16 + 4 g + 0..3) for lane group g, those are exactly the lane's
 // operand words of O^T = V^T P^T, and P never leaves its lane. V is transposed
 // into LDS in that key order while it is staged (8 keys x 8 dims a thread).
-// q and p are two fp16 terms each (22 bits), K and V fp16 as the cache holds
-// them, sums fp32. Two waves a SIMD (a lone wave issues a vector instruction
+// K and V are fp16 as the cache holds them. q and p are two fp16 terms each
+// (22 bits), which costs accuracy that the sums win back: the matrix units round
+// at the running sum's size several times an instruction, so scores are formed
+// over 64 dims at a time, low terms first, and the values of a step on their own,
+// and both are added in fp32; the exponent is one fused multiply-add of the
+// score. Distance from float64 of the same q and cache, against the token steps'
+// attention (fp32 q and p) on the same rows: 32 rows 8.9e-8 (9.3e-8), 2000 rows
+// 1.36e-7 (1.40e-7), in a window of 512 1.40e-7 (1.45e-7), from position 1500
+// 1.88e-7 (1.84e-7); with one chain a score and a value 1.28 to 1.79 times the
+// steps'. It takes the same time (2000 tokens 8.71 ms, 300 3.72). Two waves a SIMD (a lone wave issues a vector instruction
 // every 8 cycles), cache rows through raw buffers, one descriptor a load that
 // starts at the load's first row (scalar arithmetic only) and ends at the last
 // key: rows past it read as zeros.
@@ -755,8 +763,15 @@ __global__ __launch_bounds__(kPaThreads) void pf_attn_kernel(PfAttnArgs a) {
         qh[s] = *reinterpret_cast<const f16x8*>(a.qh + qr * 256u + s * 32 + g * 8u);
         ql[s] = *reinterpret_cast<const f16x8*>(a.ql + qr * 256u + s * 32 + g * 8u);
     }
-    const float qs = a.qscale[qr] * a.scale;
+    const float qs = a.qscale[qr] * a.scale * 1.4426950408889634f;
     const uint32_t free1 = min(first + 1u, kn);
+    // read offsets: the swizzles repeat every 2 steps of 32 dims of K and every
+    // 4 value tiles, the rest are constants
+    uint32_t ka[2], va[4];
+#pragma unroll
+    for (uint32_t i = 0; i < 2; ++i) ka[i] = (kg * 32u + n16) * 512u + ((4u * i + g) ^ (n16 & 7u)) * 16u;
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) va[i] = (16u * i + n16) * (kPaKeys * 2u) + ((kg * 4u + g) ^ pa_swz(16u * i + n16)) * 16u;
     f32x4 o[16];
 #pragma unroll
     for (int d = 0; d < 16; ++d) o[d] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -768,22 +783,26 @@ __global__ __launch_bounds__(kPaThreads) void pf_attn_kernel(PfAttnArgs a) {
         if (kt + kPaKeys < kn) load(kt + kPaKeys);
         const uint32_t kk = kt + kg * 32u;       // this wave's keys
         if (kk >= kn) continue;
-        f32x4 st[2], sl[2];
+        // 64 dims at a time, low terms first, added in fp32 pairwise: fewer
+        // roundings at the sum's size than in one chain
+        f32x4 st[2], part[2];
 #pragma unroll
-        for (int t = 0; t < 2; ++t) st[t] = sl[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        const uint32_t key0 = kg * 32u + n16;
-#pragma unroll
-        for (int s = 0; s < 8; ++s)
+        for (int s = 0; s < 8; s += 2)
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
-                const f16x8 kv = *reinterpret_cast<const f16x8*>(sm.t.k + (key0 + 16u * t) * 512u + ((4u * s + g) ^ (n16 & 7u)) * 16u);
-                st[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kv, qh[s], st[t], 0, 0, 0);
-                sl[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kv, ql[s], sl[t], 0, 0, 0);
+                f16x8 kv[2];
+#pragma unroll
+                for (int i = 0; i < 2; ++i) kv[i] = *reinterpret_cast<const f16x8*>(sm.t.k + ka[i] + 16u * 512u * t + 64u * s);
+                f32x4 h{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int i = 0; i < 2; ++i) h = __builtin_amdgcn_mfma_f32_16x16x32_f16(kv[i], ql[s + i], h, 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 2; ++i) h = __builtin_amdgcn_mfma_f32_16x16x32_f16(kv[i], qh[s + i], h, 0, 0, 0);
+                if (s == 0) st[t] = h;
+                else if (s == 2) st[t] += h;
+                else if (s == 4) part[t] = h;
+                else st[t] += part[t] + h;
             }
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) st[t][r] = (st[t][r] + sl[t][r]) * qs;
         if (kk < free0 || kk + 32u > free1) {
 #pragma unroll
             for (int t = 0; t < 2; ++t)
@@ -794,11 +813,11 @@ __global__ __launch_bounds__(kPaThreads) void pf_attn_kernel(PfAttnArgs a) {
                 }
         }
         float mx = fmaxf(fmaxf(fmaxf(st[0][0], st[0][1]), fmaxf(st[0][2], st[0][3])),
-                         fmaxf(fmaxf(st[1][0], st[1][1]), fmaxf(st[1][2], st[1][3])));
+                         fmaxf(fmaxf(st[1][0], st[1][1]), fmaxf(st[1][2], st[1][3]))) * qs;
         mx = fmaxf(mx, __shfl_xor(mx, 16, kWave));
         mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
         const float mn = fmaxf(m, mx), ms = mn == -INFINITY ? 0.0f : mn;
-        const float alpha = exp_hw(m - ms);      // 0 on the first keys
+        const float alpha = __builtin_amdgcn_exp2f(m - ms);   // 0 on the first keys
         m = mn;
         f16x8 ph, pl;
         float ps = 0.0f;
@@ -806,7 +825,7 @@ __global__ __launch_bounds__(kPaThreads) void pf_attn_kernel(PfAttnArgs a) {
         for (int t = 0; t < 2; ++t)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const float p = exp_hw(st[t][r] - ms) * kPaPScale;
+                const float p = __builtin_amdgcn_exp2f(fmaf(st[t][r], qs, -ms)) * kPaPScale;
                 ps += p;
                 const _Float16 h = _Float16(p);
                 ph[4 * t + r] = h;
@@ -817,12 +836,16 @@ __global__ __launch_bounds__(kPaThreads) void pf_attn_kernel(PfAttnArgs a) {
 #pragma unroll
             for (int d = 0; d < 16; ++d) o[d] *= alpha;
         }
+        // a step's sum is formed by itself and added in one rounding: four a
+        // step at the running sum's size, as one chain, round twice as much
 #pragma unroll
         for (int d = 0; d < 16; ++d) {
-            const uint32_t dim = 16u * d + n16;
-            const f16x8 vv = *reinterpret_cast<const f16x8*>(sm.t.v + dim * (kPaKeys * 2u) + ((kg * 4u + g) ^ pa_swz(dim)) * 16u);
-            o[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vv, ph, o[d], 0, 0, 0);
-            o[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vv, pl, o[d], 0, 0, 0);
+            const f16x8 vv = *reinterpret_cast<const f16x8*>(sm.t.v + va[d % 4] + 64u * (kPaKeys * 2u) * (d / 4));
+            f32x4 x = __builtin_amdgcn_mfma_f32_16x16x32_f16(vv, pl, f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+            x = __builtin_amdgcn_mfma_f32_16x16x32_f16(vv, ph, x, 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) o[d][r] += x[r];
+            if (d % 4 == 3) __builtin_amdgcn_sched_barrier(0);   // more reads ahead would spill
         }
     }
     // the row's sum over its four lane groups (each holds other keys)
@@ -847,7 +870,7 @@ __global__ __launch_bounds__(kPaThreads) void pf_attn_kernel(PfAttnArgs a) {
         const float Ms = M == -INFINITY ? 0.0f : M;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            f[q] = exp_hw(sm.c.m[q][r] - Ms);
+            f[q] = __builtin_amdgcn_exp2f(sm.c.m[q][r] - Ms);
             L += sm.c.l[q][r] * f[q];
         }
         float inv = nz > 1u ? 1.0f : 1.0f / L;
@@ -899,7 +922,7 @@ __global__ __launch_bounds__(256) void pf_attn_combine_kernel(PfAttnArgs a, uint
         float L = 0.0f, v[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
         for (uint32_t z = 0; z < nz; ++z) {
             const float* p = rec + (size_t(z) * 32u + r) * kPfRecord;
-            const float f = p[0] == -INFINITY ? 0.0f : exp_hw(p[0] - M);
+            const float f = p[0] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(p[0] - M);
             L += f * p[1];
             float e[8];
             ld8f(e, p + 4u + 8u * c);
