@@ -492,6 +492,33 @@ def test_gpu_batched_prefill(xp, xo, mode):
 
 
 @pytest.mark.gpu
+def test_gpu_prefill_after_embedding_upload(xp, mode):
+    """An embedding table uploaded after the first prompt is the one that every
+    later prompt reads, on the batched step (5 tokens) as on the GEMM engine
+    (40): XP_PREFILL_AUTO's KV rows and logits equal XP_PREFILL_TOKENS'."""
+    X = xp
+    print("case prefill after embedding upload", flush=True)
+    got = []
+    for pm in (X.XP_PREFILL_AUTO, X.XP_PREFILL_TOKENS):
+        cfg = cfg_small(X, n_layers=2, exec_mode=mode, prefill_mode=pm)
+        sess = X.DecodeSession(cfg)
+        sess.synthesize(9)
+        sess.prefill(np.arange(5, dtype=np.uint32))
+        sess.prefill(np.arange(30, dtype=np.uint32))
+        sess.upload(-1, X.T_EMBED, np.random.default_rng(2).normal(0, 1, (cfg.vocab, cfg.hidden)).astype(np.float32))
+        out = []
+        for n in (5, 40):
+            sess.reset()
+            sess.prefill(np.arange(100, 100 + n, dtype=np.uint32))
+            out.append(sess.last_logits().astype(np.float64))
+            out += [sess.kv_download(l, w, 0, n).view(np.float16).astype(np.float64) for l in range(2) for w in (0, 1)]
+        got.append(out)
+        sess.close()
+    for i, (a, b) in enumerate(zip(*got)):
+        assert np.abs(a - b).max() <= 1e-3 * np.abs(b).max(), i
+
+
+@pytest.mark.gpu
 def test_gpu_token_trace_timeline(xp):
     """xp_session_trace: stage ends are ordered (each stage's last finisher
     after the previous one's), every stage has working workgroups, and a

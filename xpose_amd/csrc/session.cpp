@@ -937,7 +937,8 @@ int xp_session_upload_part(xp_session* h, int layer, int tensor, size_t offset, 
     if (t == XP_T_EMBED) {
         if (!s.embed) {
             // First use: allocate the table and drop recorded graphs, whose
-            // embedding step was recorded without it.
+            // embedding step was recorded without it (the batched prefill
+            // step's among them; it is made again at its next use).
             XP_HIP(hipStreamSynchronize(s.st));
             if (hipMalloc(&s.embed, need) != hipSuccess) {
                 s.embed = nullptr;
@@ -948,6 +949,8 @@ int xp_session_upload_part(xp_session* h, int layer, int tensor, size_t offset, 
                     (void)hipGraphExecDestroy(g);
                     g = nullptr;
                 }
+            if (s.pre_step) prefill_batch_destroy(s.pre_step);
+            s.pre_step = nullptr;
             s.ta.embed_f32 = s.embed;
         }
         dst = s.embed;
