@@ -38,8 +38,10 @@ int PrefillEngine::reserve(size_t bytes) {
     if (arena) (void)hipFree(arena);
     arena = nullptr;
     arena_bytes = 0;
-    if (hipMalloc(reinterpret_cast<void**>(&arena), bytes) != hipSuccess)
+    if (hipMalloc(reinterpret_cast<void**>(&arena), bytes) != hipSuccess) {
+        arena = nullptr;
         return set_error(XP_E_NOMEM, "prefill: device memory (%zu bytes)", bytes);
+    }
     arena_bytes = bytes;
     return XP_OK;
 }
@@ -199,10 +201,15 @@ PrefillEngine* prefill_engine_create(const xp_session* s) {
     if (c.scale_fmt != XP_SCALE_F16_QUAD && c.scale_fmt != XP_SCALE_BF16_QUAD) why = "takes fp16 or bf16 quad scales";
     else if (c.head_dim != 256u || (G != 1u && G != 2u && G != 4u)) why = "takes 1, 2 or 4 query heads of 256 dims per kv head";
     else if (c.hidden % 128u || c.ffn % 128u || c.hidden > 8192u) why = "takes hidden and ffn sizes that are multiples of 128";
-    else if (hipMalloc(reinterpret_cast<void**>(&p->d_ids), size_t(c.max_seq) * 4) != hipSuccess) why = "has no device memory";
     if (why) {
         prefill_engine_destroy(p);
         set_error(XP_E_ARG, "prefill: the batched path %s", why);
+        return nullptr;
+    }
+    if (hipMalloc(reinterpret_cast<void**>(&p->d_ids), size_t(c.max_seq) * 4) != hipSuccess) {
+        p->d_ids = nullptr;
+        prefill_engine_destroy(p);
+        set_error(XP_E_NOMEM, "prefill: device memory (%u token ids)", c.max_seq);
         return nullptr;
     }
     return p;

@@ -20,6 +20,10 @@ std::vector<DeviceScratch*> g_scratch;  // indexed by device, never freed
 }  // namespace
 
 int set_error(int code, const char* fmt, ...) {
+    // HIP keeps a failure for the next hipGetLastError. It is reported here:
+    // the next launch's check must not report it again, whether the caller
+    // goes on another way (the prefill, with less memory) or comes back later.
+    if (code == XP_E_HIP || code == XP_E_NOMEM) (void)hipGetLastError();
     va_list ap;
     va_start(ap, fmt);
     std::vsnprintf(g_err, sizeof g_err, fmt, ap);
