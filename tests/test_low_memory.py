@@ -86,9 +86,30 @@ class Child:
             self.check(s, 300, want[300])
             s.close()
 
+    def once(self):
+        X, calls = self.X, self.var("alloc_calls", C.c_uint)
+        s = self.session(X.XP_PREFILL_AUTO)
+        self.prompt(s, 18)
+        made = calls.value
+        for pos0, n in ((0, 64), (0, 65), (0, 100), (0, 600), (500, 400), (0, 1000), (900, 30)):
+            s.set_position(pos0)
+            s.prefill(np.arange(n, dtype=np.uint32))
+        assert calls.value == made, (calls.value, made)
+        s.close()
+
+
+@pytest.mark.parametrize("hidden,ffn,heads,kvh", [(1152, 6912, 4, 1), (384, 640, 2, 2), (2048, 8192, 4, 2), (8192, 28672, 16, 8)])
+def test_prefill_buffers_hold_every_pass(hidden, ffn, heads, kvh):
+    """The one allocation against each row count's plans and key splits."""
+    lib, total = C.CDLL(os.path.join(ROOT, "tests", "native", "prefill_layout.so")), C.c_uint64()
+    for max_seq, rows in ((8192, 2048), (8192, 128), (300, 300), (40, 40)):
+        for n_cu in (256, 64):
+            assert lib.prefill_layout_misfit(hidden, ffn, heads, kvh, max_seq, rows, n_cu, C.byref(total)) == 0
+        assert rows < 2048 or total.value < rows * 20 * (hidden + ffn + 256 * (heads + 2 * kvh))
+
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("case", ["limits"])
+@pytest.mark.parametrize("case", ["limits", "once"])
 def test_gpu_prefill_low_memory(case):
     print(f"case prefill low memory {case}", flush=True)
     r = subprocess.run([sys.executable, "-u", os.path.abspath(__file__), case], capture_output=True, text=True, timeout=100)

@@ -4,8 +4,11 @@
 // KV rows and logits are the same to rounding.
 //
 // Plain launches on the session's stream: a stage takes about as long as its
-// launch or longer, so the host stays ahead. The buffers grow with the longest
-// chunk seen.
+// launch or longer, so the host stays ahead. The buffers are one allocation,
+// made at the first prompt for the most positions a pass can have (kPfMaxRows
+// or the session's context: 177 MB for 2048 at hidden 1152 and ffn 6912; half
+// as many while the device refuses it). No prompt allocates, frees or waits
+// after that. A first prompt of 32 tokens pays about 0.05 ms for it.
 #include "xp_internal.hpp"
 #include "xp_launch.hpp"
 
@@ -20,57 +23,100 @@ constexpr uint32_t kBlkP = 32;   // quantisation block along k
 size_t al(size_t v) { return (v + kAlignP - 1) & ~(kAlignP - 1); }
 }  // namespace
 
+// The buffers of a pass: byte offsets in the arena, and the floats that the
+// three of them take whose size depends on a plan's splits.
+struct PfLayout {
+    uint32_t rows = 0;           // most positions of a pass
+    size_t ids, x, a, asum, a2, asum2, qkv, y, qh, ql, qscale, part, total;
+    size_t qkv_floats = 0, y_floats = 0, part_floats = 0;
+};
+
 struct PrefillEngine {
     const xp_session* owner = nullptr;
     SessionWeights w{};
     hipStream_t st = nullptr;    // the owner's stream, during a run
     char* arena = nullptr;
-    size_t arena_bytes = 0;
-    uint32_t* d_ids = nullptr;   // [max_seq]
+    PfLayout lay;
 
     int chunk(const uint32_t* ids_dev, uint32_t rows, uint32_t pos0);
-    int reserve(size_t bytes);
 };
 
-int PrefillEngine::reserve(size_t bytes) {
-    if (bytes <= arena_bytes) return XP_OK;
-    XP_HIP(hipStreamSynchronize(st));
-    if (arena) (void)hipFree(arena);
-    arena = nullptr;
-    arena_bytes = 0;
-    if (hipMalloc(reinterpret_cast<void**>(&arena), bytes) != hipSuccess) {
-        arena = nullptr;
-        return set_error(XP_E_NOMEM, "prefill: device memory (%zu bytes)", bytes);
-    }
-    arena_bytes = bytes;
-    return XP_OK;
+namespace {
+
+// What a pass of `rows` positions runs: its GEMMs' plans and padded rows.
+struct PfPass {
+    PfGemmPlan q, o, g, d;
+    bool wide;                   // operand tiles of 32 rows, for the 128-row GEMM, else of 16
+    uint32_t pad;                // rows in whole operand tiles
+    size_t qkv_floats, y_floats;
+};
+PfPass plan_pass(const xp_config& c, int n_cu, uint32_t rows) {
+    const uint32_t H = c.hidden, F = c.ffn, qd = c.n_heads * c.head_dim, N = qd + 2 * c.n_kv_heads * c.head_dim;
+    PfPass p;
+    p.q = plan_pf_gemm(rows, N, H / kBlkP, false, n_cu);
+    p.o = plan_pf_gemm(rows, H, qd / kBlkP, false, n_cu);
+    p.g = plan_pf_gemm(rows, F, H / kBlkP, true, n_cu);
+    p.d = plan_pf_gemm(rows, H, F / kBlkP, false, n_cu);
+    p.wide = p.q.shape == 2;
+    p.pad = p.wide ? (rows + 31u) / 32u * 32u : (rows + 15u) / 16u * 16u;
+    p.qkv_floats = size_t(p.pad) * N * p.q.splits;
+    p.y_floats = size_t(p.pad) * H * std::max(p.o.splits, p.d.splits);
+    return p;
 }
+
+PfLayout plan_layout(const xp_config& c, int n_cu, uint32_t rows) {
+    const uint32_t H = c.hidden, F = c.ffn, qd = c.n_heads * c.head_dim;
+    PfLayout l;
+    l.rows = rows;
+    // The row counts up to hi that have as many row tiles as hi: their plans
+    // split no more than the fewest rows' (partial sums cost by the row), and
+    // hi pads to the most.
+    for (uint32_t lo = 1, hi; lo <= rows; lo = hi + 1u) {
+        hi = std::min(lo <= 32u ? 32u : lo <= 64u ? 64u : (lo + 127u) / 128u * 128u, rows);
+        const PfPass a = plan_pass(c, n_cu, lo), b = plan_pass(c, n_cu, hi);
+        const size_t pad = std::max(a.pad, b.pad);
+        l.qkv_floats = std::max({l.qkv_floats, a.qkv_floats / a.pad * pad, b.qkv_floats});
+        l.y_floats = std::max({l.y_floats, a.y_floats / a.pad * pad, b.y_floats});
+    }
+    // key splits only add workgroups up to one a CU
+    if (pf_attn_splits(1, 1, 1, c.max_seq, n_cu) > 1u) l.part_floats = size_t(std::max(n_cu, 256)) * 32u * kPfRecord;
+    size_t off = 0;
+    auto take = [&](size_t bytes) { const size_t o = off; off += al(bytes); return o; };
+    const size_t pad = (rows + 31u) / 32u * 32u;
+    l.ids = take(size_t(c.max_seq) * 4);
+    l.x = take(pad * H * 4);
+    l.a = take(pad * std::max(H, qd) * 4);
+    l.asum = take(pad * std::max(H, qd) / 8);
+    l.a2 = take(pad * F * 4);
+    l.asum2 = take(pad * F / 8);
+    l.qkv = take(l.qkv_floats * 4);
+    l.y = take(l.y_floats * 4);
+    l.qh = take(size_t(rows) * qd * 2);
+    l.ql = take(size_t(rows) * qd * 2);
+    l.qscale = take(size_t(rows) * c.n_heads * 4);
+    l.part = take(l.part_floats * 4);
+    l.total = off;
+    return l;
+}
+
+}  // namespace
 
 int PrefillEngine::chunk(const uint32_t* ids_dev, uint32_t rows, uint32_t pos0) {
     const xp_config& c = w.cfg;
     const uint32_t H = c.hidden, F = c.ffn, qd = c.n_heads * c.head_dim, kvd = c.n_kv_heads * c.head_dim;
     const uint32_t G = c.n_heads / c.n_kv_heads, N = qd + 2 * kvd;
-    // whole operand tiles: of 32 rows for the 128-row GEMM, else of 16
-    const bool wide = plan_pf_gemm(rows, H, H / kBlkP, false, w.n_cu).shape == 2;
-    const uint32_t pad = wide ? (rows + 31u) / 32u * 32u : (rows + 15u) / 16u * 16u, mt = pad / 16u;
-    const PfGemmPlan pq = plan_pf_gemm(rows, N, H / kBlkP, false, w.n_cu), po = plan_pf_gemm(rows, H, qd / kBlkP, false, w.n_cu),
-                     pg = plan_pf_gemm(rows, F, H / kBlkP, true, w.n_cu), pd = plan_pf_gemm(rows, H, F / kBlkP, false, w.n_cu);
+    const PfPass ps = plan_pass(c, w.n_cu, rows);
+    const PfGemmPlan &pq = ps.q, &po = ps.o, &pg = ps.g, &pd = ps.d;
+    const bool wide = ps.wide;
+    const uint32_t pad = ps.pad, mt = pad / 16u;
     const uint32_t zs_g = pf_attn_splits(rows, G, c.n_kv_heads, pos0 + rows, w.n_cu);
     const uint32_t loc_keys = c.sliding_window ? std::min(pos0 + rows, c.sliding_window + 32u) : pos0 + rows;
-    const uint32_t zs_l = pf_attn_splits(rows, G, c.n_kv_heads, loc_keys, w.n_cu);
-    // buffers of this chunk
-    size_t off = 0;
-    auto take = [&](size_t bytes) { const size_t o = off; off += al(bytes); return o; };
-    const size_t o_x = take(size_t(pad) * H * 4), o_a = take(size_t(pad) * std::max(H, qd) * 4),
-                 o_as = take(size_t(pad) * std::max(H, qd) / 8), o_a2 = take(size_t(pad) * F * 4),
-                 o_as2 = take(size_t(pad) * F / 8), o_qkv = take(size_t(pad) * N * 4 * pq.splits),
-                 o_y = take(size_t(pad) * H * 4 * std::max(po.splits, pd.splits)),
-                 o_qh = take(size_t(rows) * qd * 2), o_ql = take(size_t(rows) * qd * 2),
-                 o_qs = take(size_t(rows) * c.n_heads * 4),
-                 o_part = take(size_t(std::max(zs_g, zs_l)) > 1
-                                   ? size_t(c.n_kv_heads) * ((rows * G + 31u) / 32u) * std::max(zs_g, zs_l) * 32u * kPfRecord * 4
-                                   : 0);
-    if (int rc = reserve(off); rc != XP_OK) return rc;
+    const uint32_t zs_l = pf_attn_splits(rows, G, c.n_kv_heads, loc_keys, w.n_cu), zs = std::max(zs_g, zs_l);
+    const size_t part = zs > 1u ? size_t(c.n_kv_heads) * ((rows * G + 31u) / 32u) * zs * 32u * kPfRecord : 0;
+    if (rows > lay.rows || ps.qkv_floats > lay.qkv_floats || ps.y_floats > lay.y_floats || part > lay.part_floats)
+        return set_error(XP_E_NOMEM, "prefill: %u positions do not fit the buffers", rows);
+    const size_t o_x = lay.x, o_a = lay.a, o_as = lay.asum, o_a2 = lay.a2, o_as2 = lay.asum2, o_qkv = lay.qkv, o_y = lay.y,
+                 o_qh = lay.qh, o_ql = lay.ql, o_qs = lay.qscale, o_part = lay.part;
     auto f = [&](size_t o) { return reinterpret_cast<float*>(arena + o); };
     float* x = f(o_x);
     int rc;
@@ -184,16 +230,14 @@ int PrefillEngine::chunk(const uint32_t* ids_dev, uint32_t rows, uint32_t pos0) 
     return XP_OK;
 }
 
-PrefillEngine* prefill_engine_create(const xp_session* s) {
+int prefill_engine_create(const xp_session* s, PrefillEngine** out) {
+    *out = nullptr;
     PrefillEngine* p = new (std::nothrow) PrefillEngine;
-    if (!p) {
-        set_error(XP_E_NOMEM, "prefill: out of host memory");
-        return nullptr;
-    }
+    if (!p) return set_error(XP_E_NOMEM, "prefill: out of host memory");
     p->owner = s;
-    if (session_weights(s, &p->w) != XP_OK) {
+    if (int rc = session_weights(s, &p->w); rc != XP_OK) {
         delete p;
-        return nullptr;
+        return rc;
     }
     const xp_config& c = p->w.cfg;
     const uint32_t G = c.n_kv_heads && c.n_heads % c.n_kv_heads == 0 ? c.n_heads / c.n_kv_heads : 0;
@@ -201,18 +245,27 @@ PrefillEngine* prefill_engine_create(const xp_session* s) {
     if (c.scale_fmt != XP_SCALE_F16_QUAD && c.scale_fmt != XP_SCALE_BF16_QUAD) why = "takes fp16 or bf16 quad scales";
     else if (c.head_dim != 256u || (G != 1u && G != 2u && G != 4u)) why = "takes 1, 2 or 4 query heads of 256 dims per kv head";
     else if (c.hidden % 128u || c.ffn % 128u || c.hidden > 8192u) why = "takes hidden and ffn sizes that are multiples of 128";
+    else if (size_t(c.hidden) * c.ffn / 2 > 0xFFFFFFFFu || c.ffn > 1u << 24) why = "takes matrices of up to 4 GiB";
     if (why) {
-        prefill_engine_destroy(p);
-        set_error(XP_E_ARG, "prefill: the batched path %s", why);
-        return nullptr;
+        delete p;
+        return set_error(XP_E_ARG, "prefill: the batched path %s", why);
     }
-    if (hipMalloc(reinterpret_cast<void**>(&p->d_ids), size_t(c.max_seq) * 4) != hipSuccess) {
-        p->d_ids = nullptr;
-        prefill_engine_destroy(p);
-        set_error(XP_E_NOMEM, "prefill: device memory (%u token ids)", c.max_seq);
-        return nullptr;
+    // the GEMMs' byte offsets into a staged operand are 32 bits
+    const size_t k = std::max({c.hidden, c.ffn, c.n_heads * c.head_dim});
+    const uint32_t most = uint32_t(std::min<size_t>(std::min(kPfMaxRows, c.max_seq), 0xFFFFFFFFu / (k * 4u) / 32u * 32u));
+    for (uint32_t rows = most;; rows /= 2u) {
+        p->lay = plan_layout(c, p->w.n_cu, rows);
+        if (hipMalloc(reinterpret_cast<void**>(&p->arena), p->lay.total) == hipSuccess) break;
+        p->arena = nullptr;
+        const int rc = set_error(XP_E_NOMEM, "prefill: device memory (%zu bytes)", p->lay.total);
+        if (rows <= 64u) {
+            delete p;
+            return rc;
+        }
     }
-    return p;
+    clear_error();
+    *out = p;
+    return XP_OK;
 }
 
 int prefill_engine_run(PrefillEngine* p, const uint32_t* ids, uint32_t n, uint32_t pos0, hipStream_t st) {
@@ -220,17 +273,11 @@ int prefill_engine_run(PrefillEngine* p, const uint32_t* ids, uint32_t n, uint32
     // the weights as they are now: an embedding table may have been uploaded
     // since the last run
     if (int rc = session_weights(p->owner, &p->w); rc != XP_OK) return rc;
-    XP_HIP(hipMemcpyAsync(p->d_ids, ids, size_t(n) * 4, hipMemcpyHostToDevice, st));
-    uint32_t most = kPfMaxRows;
+    uint32_t* d_ids = reinterpret_cast<uint32_t*>(p->arena + p->lay.ids);
+    XP_HIP(hipMemcpyAsync(d_ids, ids, size_t(n) * 4, hipMemcpyHostToDevice, st));
     for (uint32_t c0 = 0; c0 < n;) {
-        const uint32_t rows = std::min(most, n - c0);
-        const int rc = p->chunk(p->d_ids + c0, rows, pos0 + c0);
-        if (rc == XP_E_NOMEM && rows > 64u) {
-            most = rows / 2u;   // nothing of this chunk was queued: shorter ones
-            clear_error();
-            continue;
-        }
-        if (rc != XP_OK) {
+        const uint32_t rows = std::min(p->lay.rows, n - c0);
+        if (int rc = p->chunk(d_ids + c0, rows, pos0 + c0); rc != XP_OK) {
             (void)hipStreamSynchronize(st);
             return rc;
         }
@@ -242,7 +289,6 @@ int prefill_engine_run(PrefillEngine* p, const uint32_t* ids, uint32_t n, uint32
 void prefill_engine_destroy(PrefillEngine* p) {
     if (!p) return;
     if (p->arena) (void)hipFree(p->arena);
-    if (p->d_ids) (void)hipFree(p->d_ids);
     delete p;
 }
 

@@ -1085,10 +1085,11 @@ int xp_session_prefill(xp_session* h, const uint32_t* ids, uint32_t n) {
             return s.pre_step != nullptr;
         };
         auto engine_ready = [&]() {
-            if (!s.pre && !s.pre_unavailable && !(s.pre = prefill_engine_create(h))) {
-                s.pre_unavailable = true;
-                clear_error();
-            }
+            if (!s.pre && !s.pre_unavailable)
+                if (const int e = prefill_engine_create(h, &s.pre); e != XP_OK) {
+                    s.pre_unavailable = e != XP_E_NOMEM;   // memory may be free at the next prompt
+                    clear_error();
+                }
             return s.pre != nullptr;
         };
         int rc = XP_E_NOMEM;

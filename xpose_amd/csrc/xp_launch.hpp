@@ -336,11 +336,12 @@ void prefill_batch_destroy(PrefillBatch* p);
 // ---- prompt prefill (prefill.cpp, prefill_engine.hip) ----
 // A session's prefill buffers: tokens ids[0..n) at positions pos0 .. pos0 + n
 // - 1 through every layer, up to kPfMaxRows positions a pass, on the session's
-// KV cache; writes the KV rows, no logits. create returns nullptr (error set)
-// when the shape does not fit. run queues on the session's stream `st` and does
-// not wait: ids (pinned) must stay as they are until it has.
+// KV cache; writes the KV rows, no logits. create fails with XP_E_ARG when the
+// shape does not fit, XP_E_NOMEM when the device has no room for 64 positions.
+// run queues on the session's stream `st` and does not wait: ids (pinned) must
+// stay as they are until it has.
 struct PrefillEngine;
-PrefillEngine* prefill_engine_create(const xp_session* s);
+int prefill_engine_create(const xp_session* s, PrefillEngine** out);
 int prefill_engine_run(PrefillEngine* p, const uint32_t* ids, uint32_t n, uint32_t pos0, hipStream_t st);
 void prefill_engine_destroy(PrefillEngine* p);
 constexpr uint32_t kPfMaxRows = 2048;
