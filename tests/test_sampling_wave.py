@@ -123,6 +123,30 @@ def test_gpu_softmax_and_draw_tiles(xp, xo, n, nparts):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n,nparts", [(1, 1), (15, 1), (16, 1), (17, 1), (63, 1), (64, 1), (65, 1), (80, 1), (1000, 1), (129, 2), (1000, 31)])
+def test_gpu_draw_inside_a_chain(xp, xo, n, nparts):
+    """The walk inside the chosen chain (64 elements at a time, the last few of
+    a chain one by one): targets on, before and past every element's running sum."""
+    X, L = xp, xo.lib()
+    print(f"case draw inside a chain n={n} nparts={nparts}", flush=True)
+    w = np.random.default_rng(n).random(n).astype(np.float32)
+    w[::5] = 0.0
+    ps = np.empty(nparts, np.float32)
+    L.xo_reduce_sum_partial(ps, w, n, nparts)
+    st = np.float32([0.0, 1.0])                          # u is the target itself
+    dw, dp, ds, do, di = dbuf(X, w), dbuf(X, ps), dbuf(X, st), X.DeviceBuffer(8), X.DeviceBuffer(4)
+    run = np.cumsum(w[::nparts], dtype=np.float32)
+    us = np.unique(np.concatenate([run[:3], run[14:18], run[62:66], run[-2:], np.float32([0.0, -1.0, 1e6])]))
+    for u in np.concatenate([us, np.nextafter(us, np.float32(1e9))]):
+        out, oi = np.empty(2, np.float32), np.empty(1, np.uint32)
+        L.xo_multinomial_strided(out, oi, w, ps, st, n, nparts, u)
+        X.call("xp_multinomial_strided", do.vp, di.vp, dw.vp, dp.vp, ds.vp, n, nparts, float(u), None)
+        X.synchronize()
+        assert int(di.download(np.uint32)[0]) == int(oi[0]), u
+        assert np.array_equal(do.download(np.float32), out), u
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("k", [1, 63, 64, 65, 200])
 def test_gpu_topp_and_draw_any_k(xp, xo, k):
     X, L = xp, xo.lib()

@@ -707,8 +707,8 @@ __global__ __launch_bounds__(kWave) void multinomial_sample_kernel(float* out, u
 
 // The chain whose running mass passes the target, then the element in it: the
 // sums and their order are the reference's, from LDS tiles in blocks as in
-// reduce_sum_final (4096 chains: 250 us by one thread, 31.5 as a chain of adds,
-// 20.8 so). A block added at once has no negative term: it is passed over where
+// reduce_sum_final (4096 chains of 64: 250 us by one thread, 31.5 as a chain of adds,
+// 19 so). A block added at once has no negative term: it is passed over where
 // its end has not passed the target. In one that may hold the place, sixteen
 // running sums are formed before their largest is held against the target.
 __global__ __launch_bounds__(kScThreads) void multinomial_strided_kernel(float* out, uint32_t* idx_out, const float* w,
@@ -773,23 +773,52 @@ __global__ __launch_bounds__(kScThreads) void multinomial_strided_kernel(float* 
     }
     if (threadIdx.x >= kWave) return;
     if (chain == kNone) chain = nparts - 1u;
+    // The element, 64 of the chain at a time, as the chain was found: sixteen
+    // running sums from LDS (with zeros past the chain's end, which pass no
+    // target that the last element did not), 12 ns an element on a chain of
+    // 32768; up to sixteen elements one by one from the lanes, which waits for
+    // no LDS (60 ns an element). The last element if none passes.
     uint32_t chosen = chain;
     float cw = 0.0f;
-    bool stop = false;
-    for (uint64_t b = chain; b < n && !stop; b += uint64_t(kWave) * nparts) {
+    for (uint64_t b = chain; b < n; b += uint64_t(kWave) * nparts) {
         const uint64_t e = b + uint64_t(threadIdx.x) * nparts;
         const float v = e < n ? w[e] : 0.0f;
         const uint64_t left = (uint64_t(n) - b + nparts - 1u) / nparts;
-        const uint32_t m = uint32_t(left < kWave ? left : kWave);
-        for (uint32_t j = 0; j < m; ++j) {
-            chosen = uint32_t(b + uint64_t(j) * nparts);
-            cw = lane_f(v, j);
-            cum += cw;
-            if (cum > target) {
-                stop = true;
-                break;
+        uint32_t at = uint32_t(left < kWave ? left : kWave) - 1u;
+        bool stop = false;
+        if (at < 16u) {
+            for (uint32_t j = 0, last = at; j <= last && !stop; ++j) {
+                at = j;
+                cum += lane_f(v, j);
+                stop = cum > target;
             }
+            cw = lane_f(v, at);
+        } else {
+            wave_lds_sync();
+            tile[threadIdx.x] = v;
+            wave_lds_sync();
+            for (uint32_t h = 0; h <= at && !stop; h += 16) {
+                float x[16], c[16];
+                ld16(x, tile + h);
+                c[0] = cum + x[0];
+#pragma unroll
+                for (int j = 1; j < 16; ++j) c[j] = c[j - 1] + x[j];
+                float mx = c[0];
+#pragma unroll
+                for (int j = 1; j < 16; ++j) mx = fmaxf(mx, c[j]);
+                cum = c[15];                             // not used again once one has passed
+                if (!(mx > target)) continue;
+#pragma unroll
+                for (int j = 15; j >= 0; --j)
+                    if (c[j] > target) {
+                        at = h + uint32_t(j);
+                        stop = true;
+                    }
+            }
+            cw = tile[at];
         }
+        chosen = uint32_t(b + uint64_t(at) * nparts);
+        if (stop) break;
     }
     if (threadIdx.x != 0) return;
     out[0] = float(chosen);
