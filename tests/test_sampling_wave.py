@@ -147,6 +147,52 @@ def test_gpu_draw_inside_a_chain(xp, xo, n, nparts):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n,nparts", [(16 * 300 - 1, 300), (16 * 300, 300), (24 * 300 - 1, 300), (24 * 300, 300), (131071 * 24, 131071),
+                                      (131072 * 25 + 5, 131072), (65536 * 17, 65536), (65536 * 16 + 1, 65536), (7, 1000)])
+def test_gpu_chain_partials_both_sides(xp, xo, n, nparts):
+    """Maxima and exponential sums where the kernels change over (a thread a
+    chain, sixteen a chain): bit for bit the oracle's of the device's exponentials."""
+    X, L = xp, xo.lib()
+    print(f"case chain partials n={n} nparts={nparts}", flush=True)
+    x = values("normal", n, nparts)
+    x[::97] = -INF
+    dx, dm, ds = dbuf(X, x), X.DeviceBuffer(4 * nparts), dbuf(X, np.float32([x.max(), 0.0]))
+    do, dp = X.DeviceBuffer(4 * n), X.DeviceBuffer(4 * nparts)
+    X.call("xp_reduce_max_partial", dm.vp, dx.vp, n, nparts, None)
+    X.call("xp_softmax_exp_partial", do.vp, dp.vp, dx.vp, ds.vp, n, nparts, None)
+    X.synchronize()
+    pm, want = np.empty(nparts, np.float32), np.empty(nparts, np.float32)
+    L.xo_reduce_max_partial(pm, x, n, nparts)
+    assert np.array_equal(dm.download(np.float32), pm)
+    e = do.download(np.float32)
+    assert np.allclose(e, np.exp(x.astype(np.float64) - float(x.max())), rtol=2e-6, atol=1e-30)
+    L.xo_reduce_sum_partial(want, e, n, nparts)
+    assert np.array_equal(dp.download(np.float32), want)
+
+
+@pytest.mark.gpu
+def test_gpu_chain_partials_past_2_28_chains(xp):
+    """Sixteen threads for each of 2^28 chains are more than a grid has."""
+    X = xp
+    nparts = (1 << 28) + 64
+    n = nparts + 3
+    print(f"case chain partials nparts={nparts}", flush=True)
+    dx, dm, ds = X.DeviceBuffer(4 * n), X.DeviceBuffer(4 * nparts), dbuf(X, np.float32([0.0, 0.0]))
+    dx.fill_bytes(0)
+    dm.fill_bytes(0xFF)
+    dx.upload(np.float32([5.0]), 4 * (nparts - 1))
+    X.call("xp_reduce_max_partial", dm.vp, dx.vp, n, nparts, None)
+    X.synchronize()
+    for off, want in ((0, [0.0] * 5), (4 * (nparts - 3), [0.0, 0.0, 5.0])):
+        assert np.array_equal(dm.download(np.float32, len(want), off), np.float32(want))
+    X.call("xp_softmax_exp_partial", dx.vp, dm.vp, dx.vp, ds.vp, n, nparts, None)
+    X.synchronize()
+    assert np.array_equal(dm.download(np.float32, 5), np.float32([2, 2, 2, 1, 1]))
+    assert np.array_equal(dm.download(np.float32, 2, 4 * (nparts - 3)), np.float32([1, 1]))
+    assert np.array_equal(dx.download(np.float32, 3, 4 * nparts), np.float32([1, 1, 1]))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("k", [1, 63, 64, 65, 200])
 def test_gpu_topp_and_draw_any_k(xp, xo, k):
     X, L = xp, xo.lib()

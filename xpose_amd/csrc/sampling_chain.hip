@@ -47,6 +47,41 @@ constexpr uint32_t kChainW = 16;                         // chains a workgroup
 constexpr uint32_t kChainR = kScThreads / kChainW;       // rows at a time
 constexpr uint32_t kChainU = 4;                          // rows in flight a thread
 
+// Short chains, or so many that a thread each fills the chip, need no sharing:
+// there the sixteen threads only cost launches of workgroups (and a grid has
+// less than 2^32 threads, which 2^28 chains would pass). Tiled / a thread each:
+//   maximum      65536 chains of 24  3.9 / 4.1 us, of 64  3.8 / 8.3; 262144 of 4  5.3 / 3.9, of 64  21.7 / 21.6
+//   exponentials 65536 chains of 8  5.2 / 4.2, of 24  5.8 / 6.9; 262144 of 1  13.3 / 4.2, of 32  18.1 / 15.3
+// From 131072 chains on (512 threads a CU) a thread each has the loads in
+// flight; a thread's exponentials are a serial chain besides, which that many
+// chains must be long against.
+bool max_by_thread(uint32_t n, uint32_t nparts) { return n / nparts < 24u || nparts >= 131072u; }
+bool exp_by_thread(uint32_t n, uint32_t nparts) { return n / nparts < 16u || nparts >= 4096u * uint64_t(n / nparts); }
+
+__global__ __launch_bounds__(kScThreads) void reduce_max_partial_thread_kernel(float* pmax, const float* x,
+                                                                               uint32_t n, uint32_t nparts) {
+    const uint32_t p = blockIdx.x * kScThreads + threadIdx.x;
+    if (p >= nparts) return;
+    float m = -INFINITY;
+    for (uint64_t k = p; k < n; k += nparts) m = fmaxf(m, x[k]);
+    pmax[p] = m;
+}
+
+__global__ __launch_bounds__(kScThreads) void softmax_exp_partial_thread_kernel(float* out, float* psum, const float* x,
+                                                                                const float* stats, uint32_t n,
+                                                                                uint32_t nparts) {
+    const uint32_t p = blockIdx.x * kScThreads + threadIdx.x;
+    if (p >= nparts) return;
+    const float m = stats[0];
+    float s = 0.0f;
+    for (uint64_t k = p; k < n; k += nparts) {
+        const float e = expf(x[k] - m);
+        out[k] = e;
+        s += e;
+    }
+    psum[p] = s;
+}
+
 // The maximum is the same in any order.
 __global__ __launch_bounds__(kScThreads) void reduce_max_partial_kernel(float* pmax, const float* x,
                                                                         uint32_t n, uint32_t nparts) {
@@ -1130,8 +1165,12 @@ int xp_reduce_max_partial(float* pmax, const float* x, uint32_t n, uint32_t npar
                           xp_stream stream) {
     XP_REQUIRE(pmax && x, "null pointer");
     XP_REQUIRE(n > 0 && nparts > 0, "n and nparts must be positive");
-    hipLaunchKernelGGL(reduce_max_partial_kernel, dim3(blocks(nparts, kChainW)), dim3(kScThreads),
-                       0, as_stream(stream), pmax, x, n, nparts);
+    if (max_by_thread(n, nparts))
+        hipLaunchKernelGGL(reduce_max_partial_thread_kernel, dim3(blocks(nparts, kScThreads)), dim3(kScThreads),
+                           0, as_stream(stream), pmax, x, n, nparts);
+    else
+        hipLaunchKernelGGL(reduce_max_partial_kernel, dim3(blocks(nparts, kChainW)), dim3(kScThreads),
+                           0, as_stream(stream), pmax, x, n, nparts);
     XP_SC_LAUNCH("xp_reduce_max_partial");
 }
 
@@ -1147,8 +1186,12 @@ int xp_softmax_exp_partial(float* out, float* psum, const float* x, const float*
                            uint32_t nparts, xp_stream stream) {
     XP_REQUIRE(out && psum && x && stats, "null pointer");
     XP_REQUIRE(n > 0 && nparts > 0, "n and nparts must be positive");
-    hipLaunchKernelGGL(softmax_exp_partial_kernel, dim3(blocks(nparts, kChainW)), dim3(kScThreads),
-                       0, as_stream(stream), out, psum, x, stats, n, nparts);
+    if (exp_by_thread(n, nparts))
+        hipLaunchKernelGGL(softmax_exp_partial_thread_kernel, dim3(blocks(nparts, kScThreads)), dim3(kScThreads),
+                           0, as_stream(stream), out, psum, x, stats, n, nparts);
+    else
+        hipLaunchKernelGGL(softmax_exp_partial_kernel, dim3(blocks(nparts, kChainW)), dim3(kScThreads),
+                           0, as_stream(stream), out, psum, x, stats, n, nparts);
     XP_SC_LAUNCH("xp_softmax_exp_partial");
 }
 
