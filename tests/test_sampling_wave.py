@@ -59,6 +59,46 @@ def test_gpu_topk_wave_bit_exact(xp, xo, kind, n, nparts, k):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["normal", "few", "holes"])
+@pytest.mark.parametrize("n,nparts,k", [(4096, 256, 1), (24 * 256, 256, 1), (8 * 4096, 4096, 4), (8 * 4096, 4096, 8), (64 * 16384, 16384, 1),
+                                        (64 * 4096, 4096, 1), (16 * 16384 - 3, 16384, 8), (16 * 16384, 16384, 16),
+                                        (81921 * 16, 81921, 16), (81921 * 16, 81921, 40)])
+def test_gpu_topk_partial_both_sides(xp, xo, kind, n, nparts, k):
+    """Where the kernels change over: a thread a chain on the first of each
+    pair of shapes, a wave a chain on the second."""
+    X, L = xp, xo.lib()
+    print(f"case topk both sides {kind} n={n} nparts={nparts} k={k}", flush=True)
+    x = values(kind, n, n + k)
+    nc = nparts * k
+    cv, ci = np.empty(nc, np.float32), np.empty(nc, np.uint32)
+    L.xo_topk_partial(cv, ci, x, n, nparts, k)
+    dv, di, dx = X.DeviceBuffer(4 * nc), X.DeviceBuffer(4 * nc), dbuf(X, x)
+    X.call("xp_topk_partial", dv.vp, di.vp, dx.vp, n, nparts, k, None)
+    X.synchronize()
+    assert np.array_equal(di.download(np.uint32), ci)
+    assert np.array_equal(dv.download(np.float32).view(np.uint32), cv.view(np.uint32))
+
+
+@pytest.mark.gpu
+def test_gpu_topk_partial_2_26_chains(xp):
+    """A wave for each of 2^26 chains is more than a grid's threads."""
+    X = xp
+    nparts, rows = 1 << 26, 16
+    n = nparts * rows
+    print(f"case topk partial nparts={nparts}", flush=True)
+    dx, dv, di = X.DeviceBuffer(4 * n), X.DeviceBuffer(4 * nparts), X.DeviceBuffer(4 * nparts)
+    dx.fill_bytes(0)
+    dv.fill_bytes(0xFF)
+    for p, r in ((0, 3), (nparts - 1, 15), (nparts // 2, 0)):
+        dx.upload(np.float32([7.0]), 4 * (p + r * nparts))
+    X.call("xp_topk_partial", dv.vp, di.vp, dx.vp, n, nparts, 1, None)
+    X.synchronize()
+    for p, want in ((0, 3 * nparts), (nparts - 1, nparts - 1 + 15 * nparts), (nparts // 2, nparts // 2), (5, 5)):
+        assert int(di.download(np.uint32, 1, 4 * p)[0]) == want
+        assert float(dv.download(np.float32, 1, 4 * p)[0]) == (0.0 if p == 5 else 7.0)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("nc,k", [(1, 1), (64, 64), (1023, 64), (1025, 3), (16384, 64), (17409, 64), (40000, 64),
                                   (3000, 65), (300, 200)])
 def test_gpu_rank_select_any_list(xp, xo, nc, k):

@@ -12,6 +12,9 @@
 // same inputs; only exp (the device libm against llvmpipe's) can differ in the
 // last bits. What has no order (exponentials, maxima, the choice of the best k)
 // is spread over as many threads as the chip has.
+#include <algorithm>
+#include <cmath>
+
 #include "xp_device.hpp"
 #include "xp_launch.hpp"
 
@@ -27,8 +30,21 @@ constexpr uint32_t kNone = 0xFFFFFFFFu;    // unfilled candidate slot
 
 uint32_t blocks(uint32_t n, uint32_t per) { return (n - 1u) / per + 1u; }   // n > 0
 
-// topk_partial: a wave a chain or a thread a chain.
-bool topk_by_wave(uint32_t n, uint32_t nparts) { return n / nparts >= 16u || nparts <= 4096u; }
+// topk_partial: a wave a chain or a thread a chain, by their times in us
+// (measured over 1 to 128 elements, 16 to 262144 chains, k 1 to 64). A thread
+// inserts: a chain's elements in turn, each past up to k others, 81920 chains at
+// once (a workgroup's lists are 32 KiB of LDS). A wave searches, 1024 elements at
+// a time, and takes a chip's share however short its chain, less where the
+// chain is no longer than k. Thread / wave: 262144 chains of 16, k = 1 14.4 /
+// 256, k = 64 393 / 182; 4096 of 8, k = 1 4.1 / 8.0, k = 8 7.9 / 5.4; 256 of 64,
+// k = 8 49.6 / 5.6. A wave a chain stays below a grid's 2^32 threads.
+bool topk_by_wave(uint32_t n, uint32_t nparts, uint32_t k) {
+    if (nparts >= 1u << 26) return false;
+    const double rows = double(n / nparts + (n % nparts != 0u)), p = nparts;
+    const double thread = 2.0 + rows * (0.08 + 0.095 * k) * double((nparts - 1u) / 81920u + 1u);
+    const double wave = rows <= k ? 3.0 + 0.68e-3 * p : std::max(5.8, 4.8 + 0.98e-3 * p * std::ceil(rows / 1024.0));
+    return wave < thread;
+}
 
 }  // namespace
 
@@ -297,7 +313,7 @@ __global__ __launch_bounds__(kTopkThreads) void topk_partial_kernel(float* cval,
     for (uint32_t j = 0; j < k; ++j) { bv[j][t] = -INFINITY; bi[j][t] = kNone; }
     if (p >= nparts) return;
     float thr = -INFINITY;                       // bv[k - 1][t]
-    for (uint32_t e = p; e < n; e += nparts) {
+    for (uint64_t e = p; e < n; e += nparts) {
         const float v = x[e];
         if (!(v > thr)) continue;
         uint32_t j = k - 1u;
@@ -307,7 +323,7 @@ __global__ __launch_bounds__(kTopkThreads) void topk_partial_kernel(float* cval,
             --j;
         }
         bv[j][t] = v;
-        bi[j][t] = e;
+        bi[j][t] = uint32_t(e);
         thr = bv[k - 1u][t];
     }
     for (uint32_t j = 0; j < k; ++j) {
@@ -1225,9 +1241,7 @@ int xp_topk_partial(float* cval, uint32_t* cidx, const float* x, uint32_t n, uin
     XP_REQUIRE(cval && cidx && x, "null pointer");
     XP_REQUIRE(n > 0 && nparts > 0, "n and nparts must be positive");
     XP_REQUIRE(k >= 1 && k <= kTopkMax, "k=%u must be in [1, %u]", k, kTopkMax);
-    // a wave a chain, unless the chains are short and so many that a thread
-    // each fills the chip
-    if (topk_by_wave(n, nparts))
+    if (topk_by_wave(n, nparts, k))
         hipLaunchKernelGGL(topk_partial_wave_kernel, dim3(nparts), dim3(kWave), 0, as_stream(stream), cval, cidx, x,
                            n, nparts, k);
     else
