@@ -99,7 +99,7 @@ def test_gpu_topk_partial_2_26_chains(xp):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("nc,k", [(1, 1), (64, 64), (1023, 64), (1025, 3), (16384, 64), (17409, 64), (40000, 64),
+@pytest.mark.parametrize("nc,k", [(1, 1), (64, 64), (128, 20), (129, 20), (129, 64), (1023, 64), (1025, 3), (16384, 64), (17409, 64), (40000, 64),
                                   (3000, 65), (300, 200)])
 def test_gpu_rank_select_any_list(xp, xo, nc, k):
     """Lists in no order: shuffled ids, empty slots, filled -inf slots, the same
