@@ -71,7 +71,8 @@ def test_gpu_prefill_apply_any_head_dim(xp, xo):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("rows,cols", [(1, 1), (5, 63), (3, 65), (9, 513), (4, 2047), (4, 2048), (6, 2049), (2, 9000)])
+@pytest.mark.parametrize("rows,cols", [(1, 1), (5, 63), (3, 65), (9, 513), (4, 2047), (4, 2048), (6, 2049), (2, 9000),
+                                       (7, 64), (7, 128), (7, 129), (7, 257), (7, 1024), (7, 1025), (9000, 191), (9000, 192), (900, 1748)])
 def test_gpu_softmax_rows_lengths(xp, rows, cols):
     X = xp
     print(f"case softmax rows {rows} x {cols}", flush=True)

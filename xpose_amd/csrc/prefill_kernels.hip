@@ -29,8 +29,10 @@ uint32_t pf_row_blocks(size_t rows) { return uint32_t((rows + kPfWaves - 1) / kP
 
 // softmax_rows_stats (llm_sampling.cl:527-547): one wave per row, up to 2048
 // columns held in registers between the maximum and the sum, so that a row
-// is read once (4096 x 2024: 24 -> 9.9 us).
-constexpr int kSmRegs = 32;
+// is read once (4096 x 2024: 24 -> 9.9 us). A row takes the time of its
+// registers, filled or not, so it gets the next power of two of 64 columns (a
+// row of 65 to 500 in 32 registers: 4000 rows 6.0 us, in its own 3.7).
+template <int kSmRegs>
 __global__ __launch_bounds__(kPfThreads) void softmax_rows_stats_kernel(float* stats, const float* x,
                                                                        uint32_t n_rows, uint32_t n_cols) {
     const uint32_t r = blockIdx.x * kPfWaves + threadIdx.x / kWave, lane = threadIdx.x % kWave;
@@ -75,7 +77,18 @@ __global__ __launch_bounds__(kPfThreads) void softmax_rows_stats_kernel(float* s
 
 // softmax_rows_apply (llm_sampling.cl:549-556): a wave takes a run of
 // kSmRun columns of one row (no division per element to find the row; eight
-// loads in flight a lane).
+// loads in flight a lane). Where runs are mostly past the row's end, or too few
+// for the CUs, a thread takes one element. Runs / elements in us: 16000 rows of
+// 65 5.2 / 3.6, of 129 6.5 / 5.4, of 200 7.1 / 7.6; 1000 rows of 1000 4.2 / 3.6,
+// of 2024 5.1 / 5.3; 4000 rows of 2024 12.2 / 16.0.
+constexpr size_t kSmFew = 3u << 19;   // elements
+__global__ void softmax_elems_apply_kernel(float* x, const float* stats, uint32_t n_cols, size_t total) {
+    for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < total;
+         i += size_t(gridDim.x) * blockDim.x) {
+        const size_t r = i / n_cols;
+        x[i] = expf(x[i] - stats[2 * r]) / stats[2 * r + 1];
+    }
+}
 constexpr uint32_t kSmRun = 8 * kWave;
 __global__ __launch_bounds__(kPfThreads) void softmax_rows_apply_kernel(float* x, const float* stats, uint32_t n_cols,
                                                                        uint32_t runs, size_t n_runs) {
@@ -475,8 +488,17 @@ int xp_softmax_rows_stats(float* stats, const float* x, uint32_t n_rows, uint32_
                           xp_stream stream) {
     XP_REQUIRE(stats && x, "null pointer");
     XP_REQUIRE(n_rows > 0 && n_cols > 0, "empty shape %u x %u", n_rows, n_cols);
-    hipLaunchKernelGGL(softmax_rows_stats_kernel, dim3(pf_row_blocks(n_rows)), dim3(kPfThreads), 0,
-                       as_stream(stream), stats, x, n_rows, n_cols);
+    const uint32_t regs = (n_cols - 1u) / kWave + 1u;   // a lane's columns
+#define XP_SM(R)                                                                                                        \
+    hipLaunchKernelGGL(softmax_rows_stats_kernel<R>, dim3(pf_row_blocks(n_rows)), dim3(kPfThreads), 0, as_stream(stream), \
+                       stats, x, n_rows, n_cols)
+    if (regs <= 1u) XP_SM(1);
+    else if (regs <= 2u) XP_SM(2);
+    else if (regs <= 4u) XP_SM(4);
+    else if (regs <= 8u) XP_SM(8);
+    else if (regs <= 16u) XP_SM(16);
+    else XP_SM(32);
+#undef XP_SM
     return launched("xp_softmax_rows_stats");
 }
 
@@ -484,6 +506,12 @@ int xp_softmax_rows_apply(float* x, const float* stats, uint32_t n_rows, uint32_
                           xp_stream stream) {
     XP_REQUIRE(stats && x, "null pointer");
     XP_REQUIRE(n_rows > 0 && n_cols > 0, "empty shape %u x %u", n_rows, n_cols);
+    const size_t total = size_t(n_rows) * n_cols;
+    if (n_cols < 192u || total <= kSmFew) {
+        hipLaunchKernelGGL(softmax_elems_apply_kernel, dim3(pf_blocks(total)), dim3(kPfThreads), 0, as_stream(stream), x,
+                           stats, n_cols, total);
+        return launched("xp_softmax_rows_apply");
+    }
     const uint32_t runs = (n_cols - 1u) / kSmRun + 1u;
     const size_t n_runs = size_t(n_rows) * runs;
     hipLaunchKernelGGL(softmax_rows_apply_kernel, dim3(uint32_t(std::min<size_t>((n_runs + kPfWaves - 1) / kPfWaves, 65536))),
