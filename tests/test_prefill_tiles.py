@@ -26,7 +26,7 @@ def close(got, want):
     (4, 1, 256, 1, 1, 0, 0), (4, 1, 256, 1, 700, 699, 0), (4, 1, 256, 16, 64, 48, 0), (4, 1, 256, 17, 65, 48, 20),
     (4, 1, 256, 200, 200, 0, 0), (4, 1, 256, 129, 640, 511, 100), (4, 2, 128, 33, 97, 64, 0), (6, 2, 36, 50, 130, 80, 7),
     (3, 3, 64, 64, 64, 0, 1), (2, 1, 20, 5, 300, 100, 0), (1, 1, 260, 70, 71, 3, 0),
-    (8, 4, 260, 700, 400, 0, 90)])
+    (8, 4, 260, 700, 400, 0, 90), (8, 8, 64, 1, 4500, 4499, 0), (8, 8, 64, 3, 4500, 4497, 512), (8, 2, 64, 60, 2100, 2040, 0)])
 def test_gpu_prefill_scores_and_apply_tiles(xp, xo, heads, kvh, hd, nq, seq, off, window):
     X, L = xp, xo.lib()
     print(f"case prefill tiles {heads}/{kvh} hd={hd} nq={nq} seq={seq} off={off} window={window}", flush=True)

@@ -137,9 +137,9 @@ struct __attribute__((aligned(16))) AsSmem {
 // instructions that only other workgroups fill, so four share a CU. The halves
 // meet in LDS, from where a wave writes whole rows, the masks scalar but for
 // the key. A tile that the masks leave nothing of is only filled, by a workgroup
-// that has other key tiles of the row to make. The grid's x is a multiple of 8
-// row tiles, so the tiles of one row, whose runs share cache lines, are written
-// through one XCD's L2. 1024 queries over 2024 keys, window 512, 4 heads: 24 us,
+// that has other key tiles of the row to make. From 8 row tiles on the grid's x
+// is a multiple of 8, so the tiles of one row, whose runs share cache lines, are
+// written through one XCD's L2. 1024 queries over 2024 keys, window 512, 4 heads: 24 us,
 // where 64 x 64 tiles took 38, a workgroup for each 32 x 64 tile 35 and one
 // thread a score 550 (the matrix units work 8, the 33 MB out take 7).
 __global__ __launch_bounds__(kPfThreads, 4) void attention_scores_prefill_kernel(
@@ -149,7 +149,6 @@ __global__ __launch_bounds__(kPfThreads, 4) void attention_scores_prefill_kernel
     const uint32_t tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave;
     const uint32_t c32 = lane % 32u, half = lane / 32u;
     const size_t rows = size_t(group) * n_query;          // of this kv head
-    const size_t kst = size_t(kv_heads) * head_dim;
     for (uint64_t tb = uint64_t(blockIdx.y) * kAsKeys; tb < seq_len; tb += uint64_t(gridDim.y) * kAsKeys)
     for (uint32_t kvh = blockIdx.z; kvh < kv_heads; kvh += gridDim.z)
     for (size_t r0 = size_t(blockIdx.x) * kAsRows; r0 < rows; r0 += size_t(gridDim.x) * kAsRows) {
@@ -532,7 +531,10 @@ int xp_attention_scores_prefill(float* scores, const float* q, const float* kcac
                "q and kcache must be 16-byte aligned");
     const uint32_t group = n_heads / kv_heads;
     const size_t qt = (size_t(group) * n_query - 1u) / kAsRows + 1u;
-    const uint32_t gx = uint32_t(std::min<size_t>((qt + 7u) / 8u * 8u, 1u << 20)), gz = std::min(kv_heads, 65535u);
+    // fewer than 8 row tiles are not rounded up: workgroups without one would
+    // take places that the key tiles need (8 kv heads of 64, one query over 8000
+    // keys: 34 us so, 6.4 without)
+    const uint32_t gx = uint32_t(qt < 8u ? qt : std::min<size_t>((qt + 7u) / 8u * 8u, 1u << 20)), gz = std::min(kv_heads, 65535u);
     // key tiles of a row spread over as many workgroups as the CUs hold at
     // once (four each): the filled ones then cost no launch of their own
     const uint32_t gy = uint32_t(std::min<uint64_t>(std::min((seq_len - 1u) / kAsKeys + 1u, 65535u),
