@@ -1,5 +1,6 @@
 """Prompt prefill through the GEMM engine (xp_session_prefill, XP_PREFILL_AUTO,
-prompts of more than 17 tokens) against XP_PREFILL_TOKENS, the token steps that
+prompts of more than 17 tokens, and shorter ones of shapes that the batched step
+does not take) against XP_PREFILL_TOKENS, the token steps that
 tests/test_session.py holds to the oracle: every KV row the prompt appends, in
 layers below a local and a global attention, and the last logits.
 
@@ -18,7 +19,8 @@ import pytest
 SHAPES = {"gemma": dict(hidden=1152, ffn=6912, n_heads=4, n_kv_heads=1),
           "narrow": dict(hidden=512, ffn=1024, n_heads=2, n_kv_heads=1),
           "mha": dict(hidden=384, ffn=640, n_heads=2, n_kv_heads=2),
-          "wide": dict(hidden=2048, ffn=1152, n_heads=4, n_kv_heads=2)}
+          "wide": dict(hidden=2048, ffn=1152, n_heads=4, n_kv_heads=2),
+          "split": dict(hidden=2048, ffn=8192, n_heads=4, n_kv_heads=2)}   # no batched step for it
 
 
 @pytest.mark.gpu
@@ -26,7 +28,8 @@ SHAPES = {"gemma": dict(hidden=1152, ffn=6912, n_heads=4, n_kv_heads=1),
     ("gemma", 18, 0, "f16"), ("gemma", 33, 700, "bf16"), ("gemma", 34, 3, "f16"), ("gemma", 65, 0, "bf16"),
     ("gemma", 66, 500, "f16"), ("gemma", 129, 0, "f16"), ("gemma", 130, 1001, "bf16"), ("gemma", 300, 333, "f16"),
     ("gemma", 40, 3000, "f16"), ("narrow", 47, 5, "f16"), ("narrow", 258, 0, "bf16"), ("narrow", 2100, 0, "f16"),
-    ("mha", 31, 600, "f16"), ("mha", 161, 0, "f16"), ("wide", 20, 90, "f16"), ("wide", 200, 450, "bf16")])
+    ("mha", 31, 600, "f16"), ("mha", 161, 0, "f16"), ("wide", 20, 90, "f16"), ("wide", 200, 450, "bf16"),
+    ("split", 3, 0, "f16"), ("split", 17, 30, "bf16"), ("split", 40, 5, "f16")])
 def test_gpu_prefill_engine_equals_token_steps(xp, shape, tokens, start, fmt):
     X = xp
     print(f"case prefill engine {shape} tokens={tokens} start={start} {fmt}", flush=True)

@@ -829,6 +829,16 @@ PrefillBatch* prefill_batch_create(const xp_session* s) {
     SessionWeights w;
     if (session_weights(s, &w) != XP_OK) return nullptr;
     if (make_batch(s, kBatchMax, w.cfg.max_seq, true, &b) != XP_OK) return nullptr;
+    // recorded here, not at the first pass: a shape that the step's GEMMs do not
+    // take (a gate/up product they would split along k) is then one that the
+    // prefill runs another way
+    if (b->b.capture(false, &b->b.graph) != XP_OK) {
+        const std::string msg = xp_last_error();
+        release(&b->b);
+        delete b;
+        set_error(XP_E_ARG, "%s", msg.c_str());
+        return nullptr;
+    }
     PrefillBatch* p = new (std::nothrow) PrefillBatch;
     if (!p) {
         release(&b->b);
