@@ -32,3 +32,11 @@ extern "C" uint32_t prefill_layout_misfit(uint32_t hidden, uint32_t ffn, uint32_
     }
     return 0;
 }
+
+// launch_pf_prep's answer to a row count (nothing is launched for one it refuses).
+extern "C" int prefill_staging_rows(uint32_t rows_pad) {
+    xp::PfPrepArgs a{};
+    a.K = 1152;
+    a.rows_pad = rows_pad;
+    return xp::launch_pf_prep(a, nullptr);
+}

@@ -108,6 +108,13 @@ def test_prefill_buffers_hold_every_pass(hidden, ffn, heads, kvh):
         assert rows < 2048 or total.value < rows * 20 * (hidden + ffn + 256 * (heads + 2 * kvh))
 
 
+@pytest.mark.parametrize("rows", [1, 15, 17, 40, 264])
+def test_prefill_staging_takes_whole_tiles(rows):
+    """Rows that are not whole operand tiles would be updated in place twice."""
+    lib = C.CDLL(os.path.join(ROOT, "tests", "native", "prefill_layout.so"))
+    assert lib.prefill_staging_rows(rows) == -1
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("case", ["limits", "once"])
 def test_gpu_prefill_low_memory(case):

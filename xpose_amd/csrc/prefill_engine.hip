@@ -75,7 +75,7 @@ template <int NC, int RW, int W>
 __global__ __launch_bounds__(RW * W * kWave) void pf_prep_kernel(PfPrepArgs a) {
     __shared__ float red[2][RW][W];
     const uint32_t rw = threadIdx.x / (W * kWave), th = threadIdx.x % (W * kWave);
-    const uint32_t row = min(blockIdx.x * RW + rw, a.rows_pad - 1u);   // a repeated last row stores the same values
+    const uint32_t row = blockIdx.x * RW + rw;   // below rows_pad: whole workgroups of rows
     const uint32_t K = a.K, npair = K / 8;
     auto own = [&](int i) { return th + W * kWave * i < npair; };
     auto word = [&](int i) { return own(i) ? th + W * kWave * i : 0u; };
@@ -953,9 +953,11 @@ int launched(const char* who) {
 }  // namespace
 
 int launch_pf_prep(const PfPrepArgs& a, hipStream_t st) {
-    if (a.K % 128u || a.K > 8192u) return set_error(XP_E_ARG, "prefill staging: K=%u", a.K);
+    // x is updated in place, so no row may be taken twice: rows_pad is whole
+    // operand tiles of 16 rows, which every RW below divides
+    if (a.K % 128u || a.K > 8192u || a.rows_pad % 16u) return set_error(XP_E_ARG, "prefill staging: K=%u rows=%u", a.K, a.rows_pad);
 #define XP_PREP(NC, RW, W) \
-    hipLaunchKernelGGL((pf_prep_kernel<NC, RW, W>), dim3((a.rows_pad + RW - 1u) / RW), dim3(RW * W * kWave), 0, st, a)
+    hipLaunchKernelGGL((pf_prep_kernel<NC, RW, W>), dim3(a.rows_pad / RW), dim3(RW * W * kWave), 0, st, a)
     if (a.K <= 1536u) {
         if (a.rows_pad <= 256u) XP_PREP(1, 1, 3);
         else XP_PREP(3, 8, 1);
