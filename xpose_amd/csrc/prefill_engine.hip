@@ -937,8 +937,15 @@ __global__ __launch_bounds__(256) void pf_attn_combine_kernel(PfAttnArgs a, uint
     }
 }
 
-// Rows up to which the small kernel is used.
+// Rows up to which the small kernel is used: one workgroup of row tiles. With
+// the small / the 128-row kernel, 26 layers of hidden 1152: 33 rows 2.03 / 2.53
+// ms, 64 2.16 / 2.54, 65 (two workgroups of row tiles) 2.64 / 2.57; 12 layers of
+// 2048: 64 1.35 / 1.58, 65 1.66 / 1.61. Hidden 512 would gain up to 128 rows
+// (0.87 / 0.99 ms).
 constexpr uint32_t kPfSmallRows = 64;
+// Blocks of k that a wave of the small kernel takes at once (its GeGLU form with
+// four row tiles three, which is 245 of 256 registers), and its waves.
+constexpr uint32_t kPfSmallD = 5, kPfSmallWaves = 8;
 // Columns a GEMM workgroup takes: of the output, or (GeGLU) of each of the two matrices.
 uint32_t pf_gemm_cols(int shape, bool geglu) {
     return geglu ? (shape == 2 ? 64u : 32u) : (shape == 2 ? 128u : 16u);
@@ -984,9 +991,12 @@ PfGemmPlan plan_pf_gemm(uint32_t rows, uint32_t cols, uint32_t nblk, bool geglu,
     if (geglu) return p;
     const uint32_t tiles = p.m_wgs * p.n_tiles, cu = uint32_t(n_cu > 0 ? n_cu : 256);
     if (p.shape < 2) {
-        // a wave takes up to D blocks at once: as many quads a split as keep
-        // eight waves at that, unless the CUs would be over-subscribed twice
-        const uint32_t per = std::max(9u, (nq * tiles + 2u * cu - 1u) / (2u * cu));
+        // as many quads a split as keep the waves at the blocks they take at
+        // once, unless the CUs would be over-subscribed twice. One quad less a
+        // split: 12 layers of hidden 2560, ffn 10240 1.45 against 1.42 ms for 32
+        // rows, 1.93 against 1.88 for 64; of 1280, 5120 0.90 against 0.91, 1.11
+        // against 1.13; of 512, 1152 and 2048 the same.
+        const uint32_t per = std::max(kPfSmallWaves * kPfSmallD / 4u, (nq * tiles + 2u * cu - 1u) / (2u * cu));
         p.splits = (nq + per - 1u) / per;
         p.qsplit = (nq + p.splits - 1u) / p.splits;
         p.splits = (nq + p.qsplit - 1u) / p.qsplit;
@@ -1014,12 +1024,12 @@ static void gemm_launch(const PfGemmArgs& a, int shape, bool ge, hipStream_t st)
     const uint32_t nC = a.n_tiles * a.splits;
     const dim3 grid(8u * a.m_wgs * ((nC + 7u) / 8u)), blk(shape == 2 ? 256 : 512);
     if (ge) {
-        if (shape == 0) hipLaunchKernelGGL((pf_gemm_small_kernel<FMT, 2, 4, 5, true>), grid, blk, 0, st, a);
+        if (shape == 0) hipLaunchKernelGGL((pf_gemm_small_kernel<FMT, 2, 4, int(kPfSmallD), true>), grid, blk, 0, st, a);
         else if (shape == 1) hipLaunchKernelGGL((pf_gemm_small_kernel<FMT, 4, 4, 3, true>), grid, blk, 0, st, a);
         else hipLaunchKernelGGL((pf_gemm_kernel<FMT, true>), grid, blk, 0, st, a);
     } else {
-        if (shape == 0) hipLaunchKernelGGL((pf_gemm_small_kernel<FMT, 2, 1, 5, false>), grid, blk, 0, st, a);
-        else if (shape == 1) hipLaunchKernelGGL((pf_gemm_small_kernel<FMT, 4, 1, 5, false>), grid, blk, 0, st, a);
+        if (shape == 0) hipLaunchKernelGGL((pf_gemm_small_kernel<FMT, 2, 1, int(kPfSmallD), false>), grid, blk, 0, st, a);
+        else if (shape == 1) hipLaunchKernelGGL((pf_gemm_small_kernel<FMT, 4, 1, int(kPfSmallD), false>), grid, blk, 0, st, a);
         else hipLaunchKernelGGL((pf_gemm_kernel<FMT, false>), grid, blk, 0, st, a);
     }
 }
