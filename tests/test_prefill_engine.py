@@ -20,7 +20,9 @@ SHAPES = {"gemma": dict(hidden=1152, ffn=6912, n_heads=4, n_kv_heads=1),
           "narrow": dict(hidden=512, ffn=1024, n_heads=2, n_kv_heads=1),
           "mha": dict(hidden=384, ffn=640, n_heads=2, n_kv_heads=2),
           "wide": dict(hidden=2048, ffn=1152, n_heads=4, n_kv_heads=2),
-          "split": dict(hidden=2048, ffn=8192, n_heads=4, n_kv_heads=2)}   # no batched step for it
+          "split": dict(hidden=2048, ffn=8192, n_heads=4, n_kv_heads=2),   # no batched step for it
+          "h2176": dict(hidden=2176, ffn=384, n_heads=2, n_kv_heads=1), "h4096": dict(hidden=4096, ffn=384, n_heads=2, n_kv_heads=1),
+          "h4224": dict(hidden=4224, ffn=384, n_heads=2, n_kv_heads=1), "h8192": dict(hidden=8192, ffn=256, n_heads=2, n_kv_heads=1)}
 
 
 @pytest.mark.gpu
@@ -29,7 +31,9 @@ SHAPES = {"gemma": dict(hidden=1152, ffn=6912, n_heads=4, n_kv_heads=1),
     ("gemma", 66, 500, "f16"), ("gemma", 129, 0, "f16"), ("gemma", 130, 1001, "bf16"), ("gemma", 300, 333, "f16"),
     ("gemma", 40, 3000, "f16"), ("narrow", 47, 5, "f16"), ("narrow", 258, 0, "bf16"), ("narrow", 2100, 0, "f16"),
     ("mha", 31, 600, "f16"), ("mha", 161, 0, "f16"), ("wide", 20, 90, "f16"), ("wide", 200, 450, "bf16"),
-    ("split", 3, 0, "f16"), ("split", 17, 30, "bf16"), ("split", 40, 5, "f16")])
+    ("split", 3, 0, "f16"), ("split", 17, 30, "bf16"), ("split", 40, 5, "f16"),
+    ("h2176", 70, 0, "f16"), ("h4096", 130, 0, "f16"), ("h4224", 20, 7, "f16"), ("h8192", 90, 0, "f16"),
+    ("gemma", 513, 0, "f16"), ("gemma", 514, 0, "f16")])
 def test_gpu_prefill_engine_equals_token_steps(xp, shape, tokens, start, fmt):
     X = xp
     print(f"case prefill engine {shape} tokens={tokens} start={start} {fmt}", flush=True)
