@@ -444,18 +444,19 @@ def test_gpu_session_error_paths(xp):
 
 
 @pytest.mark.gpu
-def test_gpu_batched_prefill(xp, xo, mode):
+@pytest.mark.parametrize("pos0,n", [(490, 37), (0, 3), (510, 10), (505, 16), (500, 17), (498, 18)])
+def test_gpu_batched_prefill(xp, xo, mode, pos0, n):
     """xp_session_prefill with XP_PREFILL_AUTO runs the first n - 1 prompt
-    tokens through the batched step (16 positions per pass on the session's
-    KV cache): against the oracle's token-by-token prefill, every appended
-    K/V row within 1e-3 of its row's max (the batched GEMM's A operand is two
-    bf16 terms), the last logits within 1e-3; against XP_PREFILL_TOKENS the
-    same; rows past the prompt untouched. The prompt (37 tokens) is not a
-    multiple of 16 and starts at 490, so it crosses the 512-position window
-    of the local layers."""
+    tokens together: up to 16 positions in one pass of the batched step (3 to 17
+    tokens), more through the GEMM engine (18 and 37). Against the oracle's
+    token-by-token prefill, every appended K/V row within 1e-3 of its row's max
+    (the GEMMs' A operand is two bf16 terms; one float16 step of the row's
+    largest value is 0.98e-3), the last logits within 1e-3; against
+    XP_PREFILL_TOKENS the same; rows past the prompt untouched. Partly filled
+    passes and operand tiles; all but the first prompt cross the 512-position
+    window of the local layers."""
     X = xp
-    print("case batched prefill", flush=True)
-    pos0, n = 490, 37
+    print(f"case batched prefill n={n} at {pos0}", flush=True)
     kvd = 256
     outs = {}
     for pm in (X.XP_PREFILL_AUTO, X.XP_PREFILL_TOKENS):
@@ -489,6 +490,34 @@ def test_gpu_batched_prefill(xp, xo, mode):
     assert a[0] == b[0]
     ok, msg = logits_close(a[1], b[1])
     assert ok, msg
+
+
+@pytest.mark.gpu
+def test_gpu_prefill_paths_in_turn(xp, mode):
+    """Prompts that follow each other on one session and go back over each
+    other's rows, through the batched step (3 to 17 tokens) and the GEMM engine:
+    the cache and the logits are those of XP_PREFILL_TOKENS all the way."""
+    X = xp
+    print("case prefill paths in turn", flush=True)
+    r = np.random.default_rng(3)
+    turns = [(0, r.integers(0, 32768, 40)), (30, r.integers(0, 32768, 9)), (39, r.integers(0, 32768, 60)), (20, r.integers(0, 32768, 17)),
+             (37, r.integers(0, 32768, 18)), (3, r.integers(0, 32768, 3)), (55, r.integers(0, 32768, 600)), (560, r.integers(0, 32768, 12))]
+    sess = []
+    for pm in (X.XP_PREFILL_AUTO, X.XP_PREFILL_TOKENS):
+        sess.append(X.DecodeSession(cfg_small(X, n_layers=2, exec_mode=mode, prefill_mode=pm)))
+        sess[-1].synthesize(6)
+    for at, ids in turns:
+        out = []
+        for s in sess:
+            s.set_position(at)
+            s.prefill(ids.astype(np.uint32))
+            assert s.position == at + ids.size
+            out.append([s.last_logits().astype(np.float64)] +
+                       [s.kv_download(l, w, 0, at + ids.size).view(np.float16).astype(np.float64) for l in range(2) for w in (0, 1)])
+        for i, (a, b) in enumerate(zip(*out)):
+            assert np.abs(a - b).max() <= 1e-3 * np.abs(b).max(), (at, i)
+    for s in sess:
+        s.close()
 
 
 @pytest.mark.gpu
