@@ -4,9 +4,12 @@ does not take) against XP_PREFILL_TOKENS, the token steps that
 tests/test_session.py holds to the oracle: every KV row the prompt appends, in
 layers below a local and a global attention, and the last logits.
 
-Tolerance: 1e-3 of a row's largest value, the bar the batched prefill has
-against the oracle (activations as two bf16 terms, 2^-18; cache rows fp16,
-2^-11). Sizes are the edges of the engine's shapes: 32-, 64- and 128-row
+Tolerance: one float16 step of a row's largest value (2^-10, 1e-3), and of all
+rows together 2e-4 in the 2-norm. Activations are two bf16 terms, so before it
+is rounded a cache value differs by d = 2^-18 to 2^-16 of itself, and rounds to
+the other side of a 2^-11 step with probability d / 2^-11: sqrt(2^-11 d) = 4e-5 to
+9e-5 (3.5e-5 to 7.6e-5 seen). The logits, which average over many such rows,
+2e-5 (0.1e-6 to 4.2e-6 seen). Sizes are the edges of the engine's shapes: 32-, 64- and 128-row
 workgroups with one row more and one less, prompts that end in a partly filled
 tile, one that takes two chunks, spans split over workgroups, one to four
 query heads a KV head, the sliding window's edge, both scale formats."""
@@ -73,7 +76,8 @@ def test_gpu_prefill_engine_equals_token_steps(xp, shape, tokens, start, fmt):
     for i, (x, y) in enumerate(zip(a, b)):
         err = np.abs(x - y).max(axis=1)
         assert np.all(err <= 1e-3 * np.abs(y).max(axis=1)), (i, int(err.argmax()), err.max())
-    assert np.abs(la - lb).max() <= 1e-3 * np.abs(lb).max()
+        assert np.linalg.norm(x - y) <= 2e-4 * np.linalg.norm(y), i
+    assert np.abs(la - lb).max() <= 2e-5 * np.abs(lb).max()
 
 
 @pytest.mark.gpu
