@@ -1,4 +1,9 @@
 // The prompt prefill's one allocation against what its passes need, on the host.
+// Names of its own: the library's must not resolve to this copy.
+#define PrefillEngine LayoutTestEngine
+#define prefill_engine_create layout_test_engine_create
+#define prefill_engine_run layout_test_engine_run
+#define prefill_engine_destroy layout_test_engine_destroy
 #include "../../xpose_amd/csrc/prefill.cpp"
 
 // The first row count up to the layout's whose pass does not fit its buffers,

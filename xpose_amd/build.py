@@ -1,7 +1,8 @@
 """Build recipe for the native parts: libxpose.so (gfx950 HIP kernels + C ABI)
-and oracle/liboracle.so (the CPU restatement used as the test checker).
+and oracle/liboracle.so (the CPU restatement used as the test checker), with the
+tests' host helpers.
 
-Both are built in-tree so the shared objects travel with the source tree.
+All are built in-tree so the shared objects travel with the source tree.
 Usage: python -m xpose_amd.build [--lib-only | --oracle-only] [-v]
 """
 from __future__ import annotations
